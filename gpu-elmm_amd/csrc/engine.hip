@@ -460,8 +460,44 @@ struct Engine : EngineIface {
   // ELMM_ZCHUNK sets both chunk lengths)
   bool zmarch_scalar = false;
   int zchunk_scalar = 16;
-  // fused momentum tile (ELMM_MOM_TILE=32x8 / 64x8 / 64x4 fixes it)
-  int mom_tile = kMomTile64x4;
+  // fused momentum tile (ELMM_MOM_TILE=32x8 / 64x8 / 64x4 fixes it).  Not
+  // autotuned: 64x8 in FP32, 32x8 in FP64 (512x512x128: 582 us against 614
+  // (64x4) and 690 (32x8) in FP32, 1410 against 1972 (64x4) in FP64, whose
+  // 64x4 rings leave LDS for one block per CU; the same order or within 3 %
+  // on every grid down to 64^3)
+  int mom_tile = sizeof(T) == 4 ? kMomTile64x8 : kMomTile32x8;
+  // Levels a block of the z-marching kernels walks: the shortest chunk whose
+  // blocks are all resident at once (kResident blocks on 256 CUs), at most
+  // the chunk length `cap` that large grids use (zchunk, zchunk_scalar,
+  // sgs_cap; lengths fixed by the environment are used as they are).  A level
+  // costs a block about 1.1 us (FP32 momentum; 3.6 us in FP64) whatever the
+  // grid, so a small grid is as fast as its longest walk: 64^3 with 16
+  // blocks of 64 levels momentum 140 us, 512 blocks of 2 levels 13 us (FP64
+  // 234 -> 22, scalar 25 -> 8, SGS 36 -> 8); past one round of resident blocks shorter
+  // walks only add prologues (256x256x64: 16 levels 89 us, 8 levels 93, 4
+  // levels 97).
+  static int zwalk(int nz, int cap, long tiles, long resident) {
+    const long chunks = std::max(1L, resident / std::max(1L, tiles));
+    return (int)std::min<long>(cap, std::max(1L, (nz + chunks - 1) / chunks));
+  }
+  static long ntiles(int nx, int ny, int tx, int ty) { return (long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty); }
+  // resident blocks: FP32 momentum 2 blocks of 512 threads or 3 of 256 a CU,
+  // FP64 2 (its 64x4 rings leave LDS for 1); scalar and SGS 4 blocks a CU in
+  // FP32, 3 in FP64 (LDS and registers)
+  int mom_walk(int tile, int cap) const {
+    if (env_zchunk) return cap;
+    constexpr bool f32 = sizeof(T) == 4;
+    const int tx = tile == kMomTile32x8 || (tile == kMomTile64x8 && !f32) ? 32 : 64, ty = tile == kMomTile64x4 ? 4 : 8;
+    const int percu = f32 ? (tx * ty == 512 ? 2 : 3) : (tx == 64 ? 1 : 2);
+    return zwalk(cfg.nz, cap, ntiles(cfg.nx, cfg.ny, tx, ty), 256L * percu);
+  }
+  int scalar_walk(int cap) const {
+    return env_scalar_zchunk ? cap : zwalk(cfg.nz, cap, ntiles(cfg.nx, cfg.ny, 64, 4), sizeof(T) == 4 ? 1024 : 768);
+  }
+  int sgs_walk(int cap) const {
+    return env_sgs_zchunk ? cap : zwalk(cfg.nz, cap, ntiles(cfg.nx, cfg.ny, 64, 8), sizeof(T) == 4 ? 1024 : 768);
+  }
+  int sgs_cap = kSgsZChunk;
   // settings fixed by the environment are not tuned
   bool env_mom_tile = false, env_zchunk = false, env_scalar_zchunk = false, env_sgs_zchunk = false;
   bool tuned = false;
@@ -556,7 +592,7 @@ struct Engine : EngineIface {
     out->mom_ty = !fused_momentum ? 0 : mom_tile == kMomTile64x4 ? 4 : 8;
     if (sizeof(T) == 8 && mom_tile == kMomTile64x8) out->mom_tx = 32;
     out->mom_zchunk = fused_momentum ? zchunk : 0;
-    out->sgs_zchunk = g.sgs_zchunk > 0 ? g.sgs_zchunk : 26;
+    out->sgs_zchunk = sgs_cap;
     out->scalar_zchunk = zmarch_scalar ? zchunk_scalar : 0;
     out->tuned = tuned ? 1 : 0;
   }
@@ -593,8 +629,9 @@ void Engine<T>::setup_geo() {
     const char *sg = std::getenv("ELMM_SGS");
     g.sgs_cellwise = sg && std::string(sg) == "cellwise";
     const char *sz = std::getenv("ELMM_SGS_ZCHUNK");
-    g.sgs_zchunk = sz ? std::max(0, std::atoi(sz)) : 0;
-    env_sgs_zchunk = g.sgs_zchunk > 0;
+    env_sgs_zchunk = sz && std::atoi(sz) > 0;
+    if (env_sgs_zchunk) sgs_cap = std::atoi(sz);
+    g.sgs_zchunk = sgs_walk(sgs_cap);
     if (const char *mt = std::getenv("ELMM_MOM_TILE")) {
       const std::string v = mt;
       mom_tile = v == "32x8" ? kMomTile32x8 : v == "64x8" ? kMomTile64x8 : kMomTile64x4;
@@ -779,7 +816,7 @@ void Engine<T>::setup_poisson() {
   {
     // room for the most partials any SGS z chunk the tuner tries gives
     const int saved = g.sgs_zchunk;
-    if (cfg.autotune && !env_sgs_zchunk) g.sgs_zchunk = 13;
+    if (cfg.autotune && !env_sgs_zchunk) g.sgs_zchunk = sgs_walk(13);
     cfl_cap = sgs_partials(g, sgs_width);
     g.sgs_zchunk = saved;
   }
@@ -1729,8 +1766,7 @@ void Engine<T>::stage(int st, bool last) {
     const uint8_t *codes[3] = {code[0].as<uint8_t>(), code[1].as<uint8_t>(), code[2].as<uint8_t>()};
     timed(ELMM_T_MOMENTUM, [&] {
       launch_momentum_zm<T>(g, u, v, w, Visc.as<T>(), Pr.as<T>(), tslot >= 0 ? s_cur[tslot] : nullptr, mslot >= 0 ? s_cur[mslot] : nullptr, ustar, U2p,
-                            codes, sc, zchunk, mom_tile,
-                                 stream);
+                            codes, sc, mom_walk(mom_tile, zchunk), mom_tile, stream);
     });
   }
   if (!fused_momentum)
@@ -1760,8 +1796,8 @@ void Engine<T>::stage(int st, bool last) {
       timed(ELMM_T_SCALAR, [&] {
         if (zmarch_scalar)
           launch_scalar_zm(g, u, v, w, TDiff.as<T>(), s_cur[s], s_nxt[s], Sadv[s]->as<T>(), code_s.as<uint8_t>(),
-                           mask[0].as<uint8_t>(), mask[1].as<uint8_t>(), mask[2].as<uint8_t>(), sc, zchunk_scalar,
-                           stream);
+                           mask[0].as<uint8_t>(), mask[1].as<uint8_t>(), mask[2].as<uint8_t>(), sc,
+                           scalar_walk(zchunk_scalar), stream);
         else
           launch_scalar(g, u, v, w, TDiff.as<T>(), s_cur[s], s_nxt[s], Sadv[s]->as<T>(), code_s.as<uint8_t>(),
                         mask[0].as<uint8_t>(), mask[1].as<uint8_t>(), mask[2].as<uint8_t>(), sc, stream);
@@ -1930,7 +1966,7 @@ template <typename T>
 void Engine<T>::autotune() {
   tuned = true;
   const auto key = std::make_tuple((int)sizeof(T), cfg.nx, cfg.ny, cfg.nz, nsc);
-  TileChoice c{mom_tile, zchunk, g.sgs_zchunk, zchunk_scalar};
+  TileChoice c{mom_tile, zchunk, sgs_cap, zchunk_scalar};
   bool hit = false;
   {
     std::lock_guard<std::mutex> lock(g_tune_mu);
@@ -1971,7 +2007,8 @@ void Engine<T>::autotune() {
       // other flipped close choices from run to run)
       std::vector<std::pair<int, int>> cand;
       for (int t : tiles)
-        for (int ch : chunks) cand.emplace_back(t, ch);
+        for (int ch : chunks)  // chunks that a small grid shortens to the same walk are one candidate
+          if (ch == chunks[0] || mom_walk(t, ch) != mom_walk(t, chunks[0])) cand.emplace_back(t, ch);
       // Each timed launch follows the kernel that precedes it in the step
       // (the SGS z-march, which reads the same velocity fields), so the
       // caches hold what they hold in the step: timed back to back instead,
@@ -1985,8 +2022,8 @@ void Engine<T>::autotune() {
                        (double *)nullptr, 0, stream);
             HIPCHK(hipEventRecord(e0, stream));
             launch_momentum_zm<T>(g, u, v, w, Visc.as<T>(), Pr.as<T>(), tslot >= 0 ? s_cur[tslot] : nullptr,
-                                  mslot >= 0 ? s_cur[mslot] : nullptr, ustar, U2p, codes, sc0, cand[k].second,
-                                  cand[k].first, stream);
+                                  mslot >= 0 ? s_cur[mslot] : nullptr, ustar, U2p, codes, sc0,
+                                  mom_walk(cand[k].first, cand[k].second), cand[k].first, stream);
             HIPCHK(hipEventRecord(e1, stream));
             HIPCHK(hipEventSynchronize(e1));
             float one = 0;
@@ -2006,8 +2043,9 @@ void Engine<T>::autotune() {
     if (!env_sgs_zchunk && !g.sgs_cellwise && !g.variable_z && sgs_width.tab) {
       const int saved = g.sgs_zchunk;
       float best = 1e30f;
-      for (int ch : {26, 32, 16, 13}) {
-        g.sgs_zchunk = ch;
+      for (int ch : {kSgsZChunk, 32, 16, 13}) {
+        if (ch != kSgsZChunk && sgs_walk(ch) == sgs_walk(kSgsZChunk)) continue;
+        g.sgs_zchunk = sgs_walk(ch);
         const float ms = time_of([&] {
           launch_sgs(g, u, v, w, Visc.as<T>(), cfg.nu, cfg.c_smag, cfg.filter_ratio, sgs_width, cfg.sgs_model,
                      (double *)nullptr, 0, stream);
@@ -2022,9 +2060,11 @@ void Engine<T>::autotune() {
     if (zmarch_scalar && nsc > 0 && !env_scalar_zchunk) {
       float best = 1e30f;
       for (int ch : {16, 13, 26, 32}) {
+        const int walk = scalar_walk(ch);
+        if (ch != 16 && walk == scalar_walk(16)) continue;
         const float ms = time_of([&] {
           launch_scalar_zm(g, u, v, w, TDiff.as<T>(), s_cur[0], s_nxt[0], Sadv[0]->as<T>(), code_s.as<uint8_t>(),
-                           mask[0].as<uint8_t>(), mask[1].as<uint8_t>(), mask[2].as<uint8_t>(), sc0, ch, stream);
+                           mask[0].as<uint8_t>(), mask[1].as<uint8_t>(), mask[2].as<uint8_t>(), sc0, walk, stream);
         });
         if (ms < best) {
           best = ms;
@@ -2042,14 +2082,15 @@ void Engine<T>::autotune() {
   }
   mom_tile = c.mom_tile;
   zchunk = c.zchunk;
-  g.sgs_zchunk = c.sgs_zchunk;
+  sgs_cap = c.sgs_zchunk;
+  g.sgs_zchunk = sgs_walk(sgs_cap);
   zchunk_scalar = c.scalar_zchunk;
   cfl_blocks = sgs_partials(g, sgs_width);
   if (std::getenv("ELMM_TUNE_LOG"))
     std::fprintf(stderr, "[elmm tune] %dx%dx%d %s%s: momentum tile %s, z chunk %d; sgs z chunk %d; scalar z chunk %d\n",
                  cfg.nx, cfg.ny, cfg.nz, sizeof(T) == 4 ? "fp32r" : "fp64", hit ? " (cached)" : "",
                  c.mom_tile == kMomTile64x4 ? "64x4" : c.mom_tile == kMomTile32x8 ? "32x8" : "64x8", c.zchunk,
-                 c.sgs_zchunk > 0 ? c.sgs_zchunk : 26, c.scalar_zchunk);
+                 c.sgs_zchunk, c.scalar_zchunk);
 }
 
 // Steps of TMarchRK3 and the main loop's time update (src/main.f90:112-169).

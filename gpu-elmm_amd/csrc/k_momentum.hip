@@ -290,12 +290,8 @@ __global__ void __launch_bounds__(TX *TY, sizeof(T) == 4 ? 4 : 3)
 }
 
 // 64 x 4 threads, two rows each (a 64 x 8 tile: 2 % faster than one row per
-// thread; 32 x 8 and 64 x 8 threads measured slower), 32 levels per block (16
-// measured equal, 64 12 % slower in FP32: fewer blocks to hide the per-level
-// load latency)
-// z chunk of 26 levels (measured 237 -> 222 us against 32 levels with the
-// earlier 5-blocks-per-CU form; ELMM_SGS_ZCHUNK overrides)
-constexpr int kSgsTX = 64, kSgsTY = 4, kSgsRPT = 2, kSgsZChunk = 26;
+// thread; 32 x 8 and 64 x 8 threads measured slower)
+constexpr int kSgsTX = 64, kSgsTY = 4, kSgsRPT = 2;
 static int sgs_zchunk(const Geo &g) { return g.sgs_zchunk > 0 ? g.sgs_zchunk : kSgsZChunk; }
 
 static bool sgs_cellwise(const Geo &g, const SgsWidth &w) { return g.sgs_cellwise || g.variable_z || !w.tab; }

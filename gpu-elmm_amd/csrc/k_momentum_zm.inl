@@ -505,9 +505,8 @@ void launch_tile(const Geo &g, const MomZArgs<T> &a, StageConst sc, int kchunk, 
 }
 }  // namespace
 
-// Tile ids: kMomTile64x4 (default; measured 5 % faster than 32x8 in FP32 on
-// 512x512x128, equal in FP64), kMomTile32x8, kMomTile64x8 (4-byte fields
-// only: its FP64 rings take 125 KiB of LDS, one block per CU; an FP64 launch
+// Tile ids: kMomTile64x4, kMomTile32x8, kMomTile64x8 (4-byte fields only:
+// its FP64 rings take 125 KiB of LDS, one block per CU; an FP64 launch
 // asking for it runs 32x8).  The engine's autotuner times them per grid.
 template <typename T>
 void launch_momentum_zm(const Geo &g, const T *U, const T *V, const T *W, const T *Visc, const T *Pr, const T *Temp,

@@ -156,6 +156,9 @@ void launch_momentum(const Geo &g, int comp, const T *U, const T *V, const T *W,
 bool momentum_zm_supported(const Geo &g);
 size_t momentum_zm_lds_bytes(int elem);
 enum { kMomTile32x8 = 0, kMomTile64x4 = 1, kMomTile64x8 = 3 };
+// levels per block of the SGS z-march on large grids (32 measured 237 against
+// 222 us on 512x512x128 in its earlier 5-blocks-per-CU form)
+constexpr int kSgsZChunk = 26;
 template <typename T>
 void launch_momentum_zm(const Geo &g, const T *U, const T *V, const T *W, const T *Visc, const T *Pr, const T *Temp,
                         const T *Moist, T *const Us[3], T *const U2[3], const uint8_t *const code[3], StageConst sc,

@@ -438,8 +438,9 @@ typedef struct elmm_timers {
 int elmm_timers_enable(elmm_handle *h, int32_t enable);
 
 /* Tile shape (x by y columns per block) and z-chunk lengths of the
- * z-marching kernels a handle uses; tuned = 1 once the autotuner has chosen
- * them.  replaces: the tile sizes of InitTiles (src/tiling.f90:16-111). */
+ * z-marching kernels a handle uses (grids too small to fill the GPU with
+ * chunks of these lengths walk shorter ones); tuned = 1 once the autotuner
+ * has chosen them.  replaces: the tile sizes of InitTiles (src/tiling.f90:16-111). */
 typedef struct elmm_tiles {
   int32_t mom_tx, mom_ty, mom_zchunk;   /* fused momentum kernel (0: per-cell kernels) */
   int32_t sgs_zchunk, scalar_zchunk;    /* SGS and scalar z-marches (0: per-cell)      */
