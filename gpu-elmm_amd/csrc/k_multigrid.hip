@@ -87,38 +87,122 @@ __global__ void __launch_bounds__(256) k_mg_zero(double *__restrict__ a, long n)
   if (t < n) a[t] = 0.0;
 }
 
-// Line Gauss-Seidel sweep of one colour: one thread per column with (i + j)
-// & 1 == color, Thomas elimination up the column (the forward values stored
-// in place: the same colour's columns are not neighbours), then back down.
-__global__ void __launch_bounds__(256) k_mg_sweep(MgLevel L, const double *__restrict__ az,
-                                                  const double *__restrict__ den, const double *__restrict__ e,
-                                                  int color) {
-  const int half = L.nx / 2;
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= half * L.ny) return;
-  const int j = t / half + 1, ii = t - (j - 1) * half;
+// Line Gauss-Seidel sweep of one colour: Thomas elimination up every column
+// with (i + j) & 1 == color (the same colour's columns are not neighbours),
+// then back down.  The serial part is one product-sum-quotient per level; its
+// inputs h - rhs need only the other colour, so a block first forms them for
+// COLS columns and all levels with every load in flight, keeps the columns in
+// LDS for the two passes, and writes them back.  (One thread per column
+// loading as it went: 30 us a sweep of 128x64 columns of 64 levels, bound by
+// a memory round trip per four levels; staged about 10.)
+// Levels are padded to whole groups of ZB (padding: zeros, whose sweeps stay
+// zero), so the chain carries no conditions and a group's operands are
+// fetched while the previous group is worked through.
+constexpr int kMgCols = 16, kMgThreads = 256, ZB = 8;
+__host__ __device__ constexpr int mg_pad(int nz) { return (nz + ZB - 1) / ZB * ZB; }
+__global__ void __launch_bounds__(kMgThreads) k_mg_sweep(MgLevel L, const double *__restrict__ az,
+                                                         const double *__restrict__ den,
+                                                         const double *__restrict__ e, int color) {
+  extern __shared__ double hs[];  // [np][kMgCols], then az, den and e [np]
+  const int half = L.nx / 2, ncol = half * L.ny, nx = L.nx, nz = L.nz, np = mg_pad(nz);
+  double *saz = hs + np * kMgCols, *sden = saz + np, *se = sden + np;
+  const int l = threadIdx.x % kMgCols, t = blockIdx.x * kMgCols + l;
+  const int tc = min(t, ncol - 1);
+  const int j = tc / half + 1, ii = tc - (j - 1) * half;
   const int i = 2 * ii + (((j + color) & 1) ? 1 : 2);
-  const int nx = L.nx, nz = L.nz;
   const long plane = (long)nx * L.ny;
   const long c = (i - 1) + (long)(j - 1) * nx;
-  const long w = (wrap_lo(i, nx) - 1) + (long)(j - 1) * nx, ea = (wrap_hi(i, nx) - 1) + (long)(j - 1) * nx;
-  const long so = (i - 1) + (long)(wrap_lo(j, L.ny) - 1) * nx, no = (i - 1) + (long)(wrap_hi(j, L.ny) - 1) * nx;
   double *P = L.phi;
-  const double *R = L.rhs;
-  double gv = 0;
-#pragma unroll 4
-  for (int k = 1; k <= nz; k++) {
-    const long o = (long)(k - 1) * plane;
-    const double h = L.ax * (P[w + o] + P[ea + o]) + L.ay * (P[so + o] + P[no + o]);
-    gv = ((h - R[c + o]) + az[k - 1] * gv) / den[k - 1];
-    P[c + o] = gv;
+  {
+    const double *R = L.rhs + c;
+    const double *W = P + (wrap_lo(i, nx) - 1) + (long)(j - 1) * nx, *E = P + (wrap_hi(i, nx) - 1) + (long)(j - 1) * nx;
+    const double *S = P + (i - 1) + (long)(wrap_lo(j, L.ny) - 1) * nx, *N = P + (i - 1) + (long)(wrap_hi(j, L.ny) - 1) * nx;
+    // the loads in batches without conditions (levels clamped into the
+    // column), so that a batch is in flight together
+    constexpr int SK = kMgThreads / kMgCols, NK = 4;
+    for (int k0 = threadIdx.x / kMgCols; k0 < np; k0 += SK * NK) {
+      double w[NK], ea[NK], so[NK], no[NK], r[NK];
+#pragma unroll
+      for (int u = 0; u < NK; u++) {
+        const long o = (long)min(k0 + u * SK, nz - 1) * plane;
+        w[u] = W[o];
+        ea[u] = E[o];
+        so[u] = S[o];
+        no[u] = N[o];
+        r[u] = R[o];
+      }
+#pragma unroll
+      for (int u = 0; u < NK; u++) {
+        const int k = k0 + u * SK;
+        const double h = L.ax * (w[u] + ea[u]) + L.ay * (so[u] + no[u]);
+        if (k < np) hs[k * kMgCols + l] = k < nz ? h - r[u] : -0.0;
+      }
+    }
+    for (int k = threadIdx.x; k < np; k += kMgThreads) {
+      const int kc = min(k, nz - 1);
+      const double a = az[kc], d = den[kc], ek = e[kc];
+      saz[k] = k < nz ? a : 0.0;
+      sden[k] = k < nz ? d : 1.0;
+      se[k] = k < nz ? ek : 0.0;
+    }
   }
-  double x = gv;
+  __syncthreads();
+  if (threadIdx.x < kMgCols) {
+    double *x = hs + l;
+    double xc[ZB], ac[ZB], dc[ZB];
+    double gv = 0;
+    auto fetch = [&](int k0, const double *p, double *xo, double *ao) {
+#pragma unroll
+      for (int b = 0; b < ZB; b++) {
+        xo[b] = x[(k0 + b) * kMgCols];
+        ao[b] = p[k0 + b];
+      }
+    };
+    fetch(0, saz, xc, ac);
+#pragma unroll
+    for (int b = 0; b < ZB; b++) dc[b] = sden[b];
+    for (int k0 = 0; k0 < np; k0 += ZB) {
+      double xn[ZB], an[ZB], dn[ZB];
+      const int kn = min(k0 + ZB, np - ZB);
+      fetch(kn, saz, xn, an);
+#pragma unroll
+      for (int b = 0; b < ZB; b++) dn[b] = sden[kn + b];
+#pragma unroll
+      for (int b = 0; b < ZB; b++) {
+        gv = (xc[b] + ac[b] * gv) / dc[b];
+        x[(k0 + b) * kMgCols] = gv;
+      }
+#pragma unroll
+      for (int b = 0; b < ZB; b++) {
+        xc[b] = xn[b];
+        ac[b] = an[b];
+        dc[b] = dn[b];
+      }
+    }
+    // P of the top level is its g: e is 0 there, and v = -0 above it leaves
+    // any sum unchanged
+    for (int k = nz; k < np; k++) x[k * kMgCols] = -0.0;
+    double v = -0.0;
+    fetch(np - ZB, se, xc, ac);
+    for (int k0 = np - ZB; k0 >= 0; k0 -= ZB) {
+      double xn[ZB], an[ZB];
+      fetch(max(k0 - ZB, 0), se, xn, an);
+#pragma unroll
+      for (int b = ZB - 1; b >= 0; b--) {
+        v = xc[b] + ac[b] * v;
+        x[(k0 + b) * kMgCols] = v;
+      }
+#pragma unroll
+      for (int b = 0; b < ZB; b++) {
+        xc[b] = xn[b];
+        ac[b] = an[b];
+      }
+    }
+  }
+  __syncthreads();
+  if (t < ncol) {
 #pragma unroll 4
-  for (int k = nz - 1; k >= 1; k--) {
-    const long o = (long)(k - 1) * plane;
-    x = P[c + o] + e[k - 1] * x;
-    P[c + o] = x;
+    for (int k = threadIdx.x / kMgCols; k < nz; k += kMgThreads / kMgCols) P[c + (long)k * plane] = hs[k * kMgCols + l];
   }
 }
 
@@ -296,7 +380,9 @@ void launch_mg_zero(double *a, long n, hipStream_t st) {
 void launch_mg_sweep(const MgLevel &L, const double *az, const double *den, const double *e, int color,
                      hipStream_t st) {
   const long cols = (long)(L.nx / 2) * L.ny;
-  hipLaunchKernelGGL(k_mg_sweep, dim3(nblk(cols, 256)), dim3(256), 0, st, L, az, den, e, color);
+  const size_t sh = (size_t)mg_pad(L.nz) * (kMgCols + 3) * sizeof(double);
+  if (sh > 65536) (void)lds_limit_raise((const void *)k_mg_sweep, sh);
+  hipLaunchKernelGGL(k_mg_sweep, dim3(nblk(cols, kMgCols)), dim3(kMgThreads), sh, st, L, az, den, e, color);
 }
 
 int mg_resmax_blocks(const MgLevel &L) { return (int)nblk((long)L.nx * L.ny * L.nz, 256); }
