@@ -97,6 +97,9 @@ int build_solids_device(const elmm_config &c, const Grid1D &g, int ncub, const e
 // Runs f(0) .. f(n-1) on n threads (f(0) on the caller's) and joins them; an
 // exception in a task is rethrown after every task has finished.
 void run_tasks(int n, const std::function<void(int)> &f);
+// Whether a spectral plan of ny rows of Mp modes and nz levels keeps a table
+// of pivot reciprocals for its z solve (k_pressure.hip).
+bool z_table_wanted(int Mp, int ny, int nz);
 // The calling thread's current HIP device, and making d current on it (the
 // server's worker threads run on the device the server was created on).
 // Defined in engine.hip.

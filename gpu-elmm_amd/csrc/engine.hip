@@ -426,7 +426,7 @@ struct Engine : EngineIface {
   DevBuf null_ijk[3];
   int null_n[3] = {0, 0, 0};
   // pressure
-  DevBuf X, twx, twy, lamx, lamy, az64, cz64;
+  DevBuf X, twx, twy, lamx, lamy, az64, cz64, zinv;
   PoissonPlan<T> pp{};
   // precision form without refinement sweeps: the spectral solve runs in
   // FP64 (complex double array) on the FP32 fields' FP64 divergence
@@ -811,6 +811,12 @@ void Engine<T>::setup_poisson() {
   // ELMM_ZPIPE=0/1 forces the z solve's load pipelining off/on (default: on
   // for grids with more than 1024 wavefronts of modes)
   if (const char *zp = std::getenv("ELMM_ZPIPE")) pp.zpipe = pp64.zpipe = std::atoi(zp) ? 1 : 0;
+  if (!use_mg && pp.zpipe < 0 && z_table_wanted(Mp, ny, nz)) {
+    zinv.alloc((size_t)Mp * ny * nz * sizeof(double));
+    launch_z_pivots(nz, ny, M, Mp, lamx.as<double>(), lamy.as<double>(), az64.as<double>(), cz64.as<double>(),
+                    zinv.as<double>(), nullptr);
+    pp.zinv = pp64.zinv = zinv.as<double>();
+  }
   top_blocks = (int)((nx * ny + 255) / 256);
   red_blocks = (int)(((long)nx * ny * nz + 255) / 256);
   {

@@ -467,6 +467,197 @@ __global__ void __launch_bounds__(64) k_solve_z(PoissonPlan<R> pp) {
   }
 }
 
+// The pivots' reciprocals 1/(b - a c') of every mode depend on the grid
+// only: the table inv[k][slot] (slots as in a level of the spectral array;
+// padding slots stay 0), by the elimination's own operations.
+__global__ void __launch_bounds__(64)
+    k_z_pivots(int nz, int ny, int M, int Mp, const double *__restrict__ lamx, const double *__restrict__ lamy,
+               const double *__restrict__ az, const double *__restrict__ cz, double *__restrict__ inv) {
+  const long plane = (long)ny * Mp, q = (long)blockIdx.x * 64 + threadIdx.x;
+  if (q >= plane) return;
+  const int m = (int)(q % Mp), j = (int)(q / Mp);
+  if (m >= M || q == 0) return;
+  const double lam = lamx[m] + lamy[j];
+  double cp = 0;
+  for (int k = 0; k < nz; k++) {
+    const double a = az[k], c = cz[k];
+    const double b = lam - a - c;
+    const double r = 1.0 / (b - a * cp);
+    cp = c * r;
+    inv[(long)k * plane + q] = r;
+  }
+}
+
+// Pass 3 with the table of pivot reciprocals: the elimination's serial chain
+// is then one product-difference-product per level instead of a division
+// (same operations on the same operands, so the same bits as k_solve_z), and
+// the real and imaginary parts are independent.  A block stages its columns
+// (ZL reals: ZL/2 modes, all levels), their pivots and the z coefficients in
+// LDS with every load in flight at once, ZL threads run the two sweeps there,
+// and all threads write the columns back: the spectral array is read and
+// written once.  Levels are padded to whole groups of ZB with zeros (whose
+// elimination gives zeros), so the chain carries no conditions and a group's
+// operands are fetched while the previous group is worked through.
+// Measured against k_solve_z (us with event overhead): 64^3 38 -> 12,
+// 144x144x72 44 -> 17, 256x128x128 80 -> 37, 256x256x128 92 -> 58, but
+// 512x256x128 105 -> 101 and 512x512x128 155 -> 188 (there k_solve_z streams
+// at 4.8 TB/s and the table adds a third of traffic): used up to 1024
+// wavefronts of modes.  ZL = 16 and 64 are slower (256x128x128: 47 and 49).
+constexpr int ZL = 32, ZB = 8, kZThreads = 256;
+
+__host__ __device__ constexpr int z_pad(int nz) { return (nz + ZB - 1) / ZB * ZB; }
+__host__ __device__ constexpr size_t solve_z_table_lds(int nz) {
+  return (size_t)z_pad(nz) * (ZL + ZL / 2 + 4) * sizeof(double);
+}
+
+template <typename R>
+__global__ void __launch_bounds__(kZThreads) k_solve_z_table(PoissonPlan<R> pp) {
+  extern __shared__ double zlds[];
+  const int nz = pp.nz, np = z_pad(nz), t = threadIdx.x;
+  double *xs = zlds, *iv = xs + np * ZL, *az = iv + np * (ZL / 2), *cz = az + np, *gm = cz + np;
+  const long plane = (long)pp.ny * pp.Mp, w2 = 2 * plane;
+  const long q0 = (long)blockIdx.x * ZL;
+  R *X = reinterpret_cast<R *>(pp.X);
+  {
+    // the loads in batches without conditions (levels clamped into the
+    // column), so that a batch is in flight together
+    constexpr int SX = kZThreads / ZL, SP = 2 * SX, NX = 16, NP = 8;
+    static_assert(SX * NX == SP * NP, "both batches cover the same levels");
+    const int l = t % ZL, lp = t % (ZL / 2), kx = t / ZL, kp = t / (ZL / 2);
+    const R *src = X + min(q0 + l, w2 - 1);
+    const double *tab = pp.zinv + min(q0 / 2 + lp, plane - 1);
+    for (int k0 = 0; k0 < np; k0 += SX * NX) {
+      R v[NX];
+      double p[NP];
+#pragma unroll
+      for (int u = 0; u < NX; u++) v[u] = src[(long)min(k0 + kx + u * SX, nz - 1) * w2];
+#pragma unroll
+      for (int u = 0; u < NP; u++) p[u] = tab[(long)min(k0 + kp + u * SP, nz - 1) * plane];
+#pragma unroll
+      for (int u = 0; u < NX; u++) {
+        const int k = k0 + kx + u * SX;
+        if (k < np) xs[k * ZL + l] = k < nz ? (double)v[u] : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < NP; u++) {
+        const int k = k0 + kp + u * SP;
+        if (k < np) iv[k * (ZL / 2) + lp] = k < nz ? p[u] : 0.0;
+      }
+    }
+    for (int k = t; k < np; k += kZThreads) {
+      const double a = pp.az[min(k, nz - 1)], c = pp.cz[min(k, nz - 1)];
+      az[k] = k < nz ? a : 0.0;
+      cz[k] = k < nz ? c : 0.0;
+    }
+  }
+  __syncthreads();
+  if (t < ZL && q0 + t >= 2) {
+    double *x = xs + t;
+    const double *r = iv + t / 2;
+    double xc[ZB], rc[ZB], ac[ZB];
+    auto fetch = [&](int k0, const double *coef, double *xo, double *ro, double *ao) {
+#pragma unroll
+      for (int e = 0; e < ZB; e++) {
+        xo[e] = x[(k0 + e) * ZL];
+        ro[e] = r[(k0 + e) * (ZL / 2)];
+        ao[e] = coef[k0 + e];
+      }
+    };
+    double d = 0;
+    fetch(0, az, xc, rc, ac);
+    for (int k0 = 0; k0 < np; k0 += ZB) {
+      double xn[ZB], rn[ZB], an[ZB];
+      fetch(min(k0 + ZB, np - ZB), az, xn, rn, an);
+#pragma unroll
+      for (int e = 0; e < ZB; e++) {
+        d = (xc[e] - ac[e] * d) * rc[e];
+        x[(k0 + e) * ZL] = d;
+      }
+#pragma unroll
+      for (int e = 0; e < ZB; e++) {
+        xc[e] = xn[e];
+        rc[e] = rn[e];
+        ac[e] = an[e];
+      }
+    }
+    double v = 0;
+    fetch(np - ZB, cz, xc, rc, ac);
+    for (int k0 = np - ZB; k0 >= 0; k0 -= ZB) {
+      double xn[ZB], rn[ZB], an[ZB], cp[ZB];
+      fetch(max(k0 - ZB, 0), cz, xn, rn, an);
+#pragma unroll
+      for (int e = 0; e < ZB; e++) cp[e] = ac[e] * rc[e];
+#pragma unroll
+      for (int e = ZB - 1; e >= 0; e--) {
+        v = xc[e] - cp[e] * v;
+        x[(k0 + e) * ZL] = v;
+      }
+#pragma unroll
+      for (int e = 0; e < ZB; e++) {
+        xc[e] = xn[e];
+        rc[e] = rn[e];
+        ac[e] = an[e];
+      }
+    }
+  } else if (q0 == 0 && t >= 64 && t < 66) {
+    // the horizontal-mean mode (see k_solve_z), its two parts by two threads
+    // of a wavefront of their own
+    // (padding levels add -0 to a zero sum)
+    double *x = xs + (t - 64), *g = gm + (t - 64) * np;
+    double xc[ZB], hc[ZB], G = 0, c = 0;
+    auto fetch = [&](int k0, const double *src, int stride, const double *h, int first, double *xo, double *ho) {
+#pragma unroll
+      for (int e = 0; e < ZB; e++) {
+        xo[e] = src[(k0 + e) * stride];
+        ho[e] = h[min(k0 + e + first, nz)];
+      }
+    };
+    fetch(np - ZB, x, ZL, pp.dzPr, 1, xc, hc);
+    for (int k0 = np - ZB; k0 >= 0; k0 -= ZB) {
+      double xn[ZB], hn[ZB];
+      fetch(max(k0 - ZB, 0), x, ZL, pp.dzPr, 1, xn, hn);
+#pragma unroll
+      for (int e = ZB - 1; e >= 0; e--) {  // (the sum past level 0 is not used)
+        const double tt = -xc[e] * hc[e], y = tt - c, s2 = G + y;
+        c = (s2 - G) - y;
+        G = s2;
+        g[k0 + e] = G;
+      }
+#pragma unroll
+      for (int e = 0; e < ZB; e++) {
+        xc[e] = xn[e];
+        hc[e] = hn[e];
+      }
+    }
+    double v = 0;
+    c = 0;
+    fetch(0, g, 1, pp.dzW, 0, xc, hc);
+    xc[0] = 0;  // x_1 = 0
+    for (int k0 = 0; k0 < np; k0 += ZB) {
+      double xn[ZB], hn[ZB];
+      fetch(min(k0 + ZB, np - ZB), g, 1, pp.dzW, 0, xn, hn);
+#pragma unroll
+      for (int e = 0; e < ZB; e++) {
+        const double tt = xc[e] * hc[e], y = tt - c, s2 = v + y;
+        c = (s2 - v) - y;
+        v = s2;
+        x[(k0 + e) * ZL] = v;
+      }
+#pragma unroll
+      for (int e = 0; e < ZB; e++) {
+        xc[e] = xn[e];
+        hc[e] = hn[e];
+      }
+    }
+  }
+  __syncthreads();
+  const int l = t % ZL;
+  if (q0 + l < w2) {
+#pragma unroll 8
+    for (int k = t / ZL; k < nz; k += kZThreads / ZL) X[(long)k * w2 + q0 + l] = (R)xs[k * ZL + l];
+  }
+}
+
 // Pass 5: inverse x FFT from the half spectrum (Hermitian symmetry), real
 // part scaled by 1/(nx*ny) -> Phi interior (FP64); with accumulate the
 // result is added to Phi (iterative-refinement correction).
@@ -595,8 +786,24 @@ void launch_fft_y(const PoissonPlan<R> &pp, int inverse, hipStream_t st) {
   });
 }
 
+bool z_table_wanted(int Mp, int ny, int nz) {
+  return ((long)Mp * ny + 63) / 64 <= 1024 && solve_z_table_lds(nz) <= 160 * 1024;
+}
+
+void launch_z_pivots(int nz, int ny, int M, int Mp, const double *lamx, const double *lamy, const double *az,
+                     const double *cz, double *inv, hipStream_t st) {
+  hipLaunchKernelGGL(k_z_pivots, dim3(nblk((long)ny * Mp, 64)), dim3(64), 0, st, nz, ny, M, Mp, lamx, lamy, az, cz,
+                     inv);
+}
+
 template <typename R>
 void launch_poisson_solve_z(const Geo &, const PoissonPlan<R> &pp, hipStream_t st) {
+  if (pp.zinv) {
+    const size_t sh = solve_z_table_lds(pp.nz);
+    allow_lds((const void *)k_solve_z_table<R>, sh);
+    hipLaunchKernelGGL(k_solve_z_table<R>, dim3(nblk(2L * pp.Mp * pp.ny, ZL)), dim3(kZThreads), sh, st, pp);
+    return;
+  }
   // nz <= kSolveZMaxNz is checked when the plan is set up
   const long modes = (long)pp.Mp * pp.ny;
   const unsigned blocks = (unsigned)((modes + 63) / 64);

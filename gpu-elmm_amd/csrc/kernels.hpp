@@ -221,7 +221,11 @@ struct PoissonPlan {
   const double *az, *cz;        // z coupling coefficients per k (0-based)
   const double *dzPr, *dzW;     // grid spacings indexed like the reference (k = 1..nz)
   int zpipe = -1;               // z solve load pipelining: -1 by grid size, 0 off, 1 on
+  const double *zinv = nullptr; // pivot reciprocals of the z solve, [nz][ny * Mp] (null: divide)
 };
+bool z_table_wanted(int Mp, int ny, int nz);
+void launch_z_pivots(int nz, int ny, int M, int Mp, const double *lamx, const double *lamy, const double *az,
+                     const double *cz, double *inv, hipStream_t st);
 template <typename T, typename R>
 void launch_fft_x_fwd(const Geo &g, const PoissonPlan<R> &pp, const T *U, const T *V, const T *W, const double *Q,
                       const uint32_t *qmask, const double *rhs, const double *phi, double dt2_rec, double *rhs_out,

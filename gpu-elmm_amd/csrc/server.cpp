@@ -161,6 +161,8 @@ int elmm_footprint(const elmm_config *cfg, int64_t *bytes) {
   } else {
     // spectral array: complex FP32 with refinement sweeps, complex FP64 otherwise
     b += (int64_t)Mp * cfg->ny * cfg->nz * 2 * es;
+    // pivot reciprocals of the z solve
+    if (elmm::z_table_wanted((int)Mp, cfg->ny, cfg->nz)) b += (int64_t)Mp * cfg->ny * cfg->nz * 8;
   }
   // block partials of the reductions (divergence, CFL, delta: at most four
   // doubles per 256 cells) and the allocation granularity of the ~60
