@@ -1672,8 +1672,10 @@ void Engine<T>::xfer_rows(E *d, const int lo[3], const int hi[3], int lb, const 
   // rows in memory order: row r holds (j, k) with r = (j + 2) + (ny + 6)(k + 2)
   const long per_k = cfg.ny + 6, r0 = (lo[1] + 2) + per_k * (lo[2] + 2), r1 = (hi[1] + 2) + per_k * (hi[2] + 2) + 1;
   const long row_bytes = g.sy * (long)sizeof(E);
-  // a thread per half MiB, at most 8 (a thread costs about 20 us to start)
-  const int nth = (int)std::min<long>(8, std::max<long>(1, (r1 - r0) * row_bytes / 524288));
+  // a thread per 2 MiB, at most 4 (per half MiB: 64^3 0.18 -> 0.3 ms a field
+  // beside a program's own busy threads; per 8 MiB: 256x128x128 1.4 -> 1.8;
+  // 512x512x128 in 2, 3, 4, 8 threads 12.3, 8.7, 7.6, 7.6)
+  const int nth = (int)std::min<long>(4, std::max<long>(1, (r1 - r0) * row_bytes / (2 << 20)));
   const long slab = std::max(1L, std::min<long>(PinnedPool::kSlotBytes / row_bytes, (r1 - r0 + nth - 1) / nth));
   const long nslab = (r1 - r0 + slab - 1) / slab;
   const int w = hi[0] - lo[0] + 1;
