@@ -120,7 +120,7 @@ __device__ inline void scalar_finish(const StageConst &sc, const Real *__restric
                                      Real *__restrict__ Sadv, long p, Real a) {
   Real s2 = sc.stage > 0 ? Sadv[p] * (Real)sc.rho_dt : (Real)0.0;
   s2 = s2 + a * (Real)sc.beta_dt;
-  Sadv[p] = a;
+  if (sc.stage < 2) Sadv[p] = a;  // the next step's first stage does not read it
   Snew[p] = S[p] + s2;
 }
 
@@ -317,7 +317,7 @@ __global__ void __launch_bounds__(NTS)
         } else {
           Real s2 = sc.stage > 0 ? cur.sadv * (Real)sc.rho_dt : (Real)0.0;
           s2 = s2 + a * (Real)sc.beta_dt;
-          Sadv[p] = a;
+          if (sc.stage < 2) Sadv[p] = a;
           Snew[p] = s0 + s2;
         }
       }
