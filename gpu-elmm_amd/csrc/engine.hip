@@ -1914,19 +1914,14 @@ void Engine<T>::stage(int st, bool last) {
   subgrid_stresses(st == 0 && (cfg.cfl_check || cfg.variable_dt));
   T *ustar[3] = {Us.as<T>(), Vs.as<T>(), Ws.as<T>()};
   T *U2p[3] = {u2, v2, w2};
-  if (fused_momentum) {
-    const uint8_t *codes[3] = {code[0].as<uint8_t>(), code[1].as<uint8_t>(), code[2].as<uint8_t>()};
-    timed(ELMM_T_MOMENTUM, [&] {
+  const uint8_t *codes[3] = {code[0].as<uint8_t>(), code[1].as<uint8_t>(), code[2].as<uint8_t>()};
+  timed(ELMM_T_MOMENTUM, [&] {
+    if (fused_momentum)
       launch_momentum_zm<T>(g, u, v, w, Visc.as<T>(), Pr.as<T>(), tslot >= 0 ? s_cur[tslot] : nullptr, mslot >= 0 ? s_cur[mslot] : nullptr, ustar, U2p,
                             codes, sc, mom_walk(mom_tile, zchunk), mom_tile, stream);
-    });
-  }
-  if (!fused_momentum)
-    for (int c = 0; c < 3; c++)
-      timed(ELMM_T_MOMENTUM, [&] {
-        launch_momentum(g, c, u, v, w, Visc.as<T>(), Pr.as<T>(), ustar[c], U2p[c], code[c].as<uint8_t>(),
-                        sc, stream);
-      });
+    else
+      launch_momentum<T>(g, u, v, w, Visc.as<T>(), Pr.as<T>(), ustar, U2p, codes, sc, stream);
+  });
   if (mom_terms[0].n + mom_terms[1].n + mom_terms[2].n) {
     // the three components' ordered corrections read only the stage-start
     // fields and write disjoint arrays: one launch

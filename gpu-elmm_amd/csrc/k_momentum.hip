@@ -997,7 +997,7 @@ __device__ inline void finish(const Geo &g, const StageConst &sc, const T *__res
       u2 = u2 + (T)sc.Az * (Pr[p + g.sz] - Pr[p]);
   }
   u2 = u2 + F[p];
-  Ustar[p] = w;
+  if (sc.stage < 2) Ustar[p] = w;  // the next step's first stage does not read it
   U2[p] = u2;
 }
 
@@ -1016,19 +1016,15 @@ __device__ inline T momentum_rhs(const Geo &g, const T *__restrict__ U, const T 
 }
 
 template <typename T, int C, int VZ>
-__global__ void __launch_bounds__(256)
-    k_momentum(Geo g, const T *__restrict__ U, const T *__restrict__ V, const T *__restrict__ W,
-               const T *__restrict__ Visc, const T *__restrict__ Pr, T *__restrict__ Ustar,
-               T *__restrict__ U2, const uint8_t *__restrict__ code, StageConst sc) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
-  const int k = blockIdx.z + 1;
-  if (i > g.n[C][0] || j > g.n[C][1]) return;
+__device__ inline void momentum_cell(const Geo &g, const T *__restrict__ U, const T *__restrict__ V,
+                                     const T *__restrict__ W, const T *__restrict__ Visc, const T *__restrict__ Pr,
+                                     T *__restrict__ Ustar, T *__restrict__ U2, uint8_t cd, const StageConst &sc,
+                                     int i, int j, int k) {
+  if (i > g.n[C][0] || j > g.n[C][1] || k > g.n[C][2]) return;
   const long p = gix(g, i, j, k);
-  const uint8_t cd = code[p];
   const T *F = C == 0 ? U : C == 1 ? V : W;
   const T w = momentum_rhs<T, C, VZ>(g, U, V, W, Visc, p, k, cd);
-  const T us_prev = Ustar[p];
+  const T us_prev = sc.stage > 0 ? Ustar[p] : (T)0;
   if (cd & CODE_CORRECTED) {
     // hand-over to the ordered-correction kernel: the bulk value in Ustar,
     // the previous stage's Ustar in U2
@@ -1040,25 +1036,34 @@ __global__ void __launch_bounds__(256)
 }
 
 template <typename T, int VZ>
-void launch_momentum_vz(const Geo &g, int comp, const T *U, const T *V, const T *W, const T *Visc, const T *Pr,
-                        T *Ustar, T *U2, const uint8_t *code, StageConst sc, hipStream_t st) {
-  const int *n = g.n[comp];
-  dim3 b(64, 4, 1), gr(nblk(n[0], 64), nblk(n[1], 4), n[2]);
-  if (comp == 0)
-    hipLaunchKernelGGL((k_momentum<T, 0, VZ>), gr, b, 0, st, g, U, V, W, Visc, Pr, Ustar, U2, code, sc);
-  else if (comp == 1)
-    hipLaunchKernelGGL((k_momentum<T, 1, VZ>), gr, b, 0, st, g, U, V, W, Visc, Pr, Ustar, U2, code, sc);
-  else
-    hipLaunchKernelGGL((k_momentum<T, 2, VZ>), gr, b, 0, st, g, U, V, W, Visc, Pr, Ustar, U2, code, sc);
+__global__ void __launch_bounds__(256)
+    k_momentum(Geo g, const T *__restrict__ U, const T *__restrict__ V, const T *__restrict__ W,
+               const T *__restrict__ Visc, const T *__restrict__ Pr, Mom3<T> m, StageConst sc) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
+  const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
+  const int k = blockIdx.z + 1;
+  if (i > g.nx || j > g.ny) return;
+  const long p = gix(g, i, j, k);
+  const uint8_t c0 = m.code[0][p], c1 = m.code[1][p], c2 = m.code[2][p];
+  momentum_cell<T, 0, VZ>(g, U, V, W, Visc, Pr, m.Us[0], m.U2[0], c0, sc, i, j, k);
+  momentum_cell<T, 1, VZ>(g, U, V, W, Visc, Pr, m.Us[1], m.U2[1], c1, sc, i, j, k);
+  momentum_cell<T, 2, VZ>(g, U, V, W, Visc, Pr, m.Us[2], m.U2[2], c2, sc, i, j, k);
 }
 
 template <typename T>
-void launch_momentum(const Geo &g, int comp, const T *U, const T *V, const T *W, const T *Visc, const T *Pr, T *Ustar,
-                     T *U2, const uint8_t *code, StageConst sc, hipStream_t st) {
+void launch_momentum(const Geo &g, const T *U, const T *V, const T *W, const T *Visc, const T *Pr, T *const Us[3],
+                     T *const U2[3], const uint8_t *const code[3], StageConst sc, hipStream_t st) {
+  Mom3<T> m;
+  for (int c = 0; c < 3; c++) {
+    m.Us[c] = Us[c];
+    m.U2[c] = U2[c];
+    m.code[c] = code[c];
+  }
+  dim3 b(64, 4, 1), gr(nblk(g.nx, 64), nblk(g.ny, 4), g.nz);
   if (g.variable_z)
-    launch_momentum_vz<T, 1>(g, comp, U, V, W, Visc, Pr, Ustar, U2, code, sc, st);
+    hipLaunchKernelGGL((k_momentum<T, 1>), gr, b, 0, st, g, U, V, W, Visc, Pr, m, sc);
   else
-    launch_momentum_vz<T, 0>(g, comp, U, V, W, Visc, Pr, Ustar, U2, code, sc, st);
+    hipLaunchKernelGGL((k_momentum<T, 0>), gr, b, 0, st, g, U, V, W, Visc, Pr, m, sc);
 }
 
 // Cells with wall-model face-flux replacements (wmfluxes-nobranch-inc.f90:
@@ -1150,6 +1155,12 @@ void launch_momentum_corr3(const Geo &g, const T *U, const T *V, const T *W, con
   else
     hipLaunchKernelGGL((k_momentum_corr3<T, 0>), dim3(nblk(tot, 128)), dim3(128), 0, st, g, U, V, W, Visc, Pr, a, sc,
                        fluxp, fluxm);
+template <typename T>
+struct Mom3 {
+  T *Us[3], *U2[3];
+  const uint8_t *code[3];
+};
+
 }
 
 template <typename T, int VZ>
@@ -1375,8 +1386,8 @@ void launch_mass_sources(const Geo &g, TermList tl, const T *U, const T *V, cons
                                     double, int, hipStream_t);                                                     \
   template void launch_wm_ustar<T>(const Geo &, const T *, const T *, const T *, const T *, const T *,             \
                                    WMUstarPoints, double, T *, hipStream_t);                                       \
-  template void launch_momentum<T>(const Geo &, int, const T *, const T *, const T *, const T *, const T *, T *,   \
-                                   T *, const uint8_t *, StageConst, hipStream_t);                                 \
+  template void launch_momentum<T>(const Geo &, const T *, const T *, const T *, const T *, const T *,            \
+                                   T *const[3], T *const[3], const uint8_t *const[3], StageConst, hipStream_t);   \
   template void launch_momentum_corr3<T>(const Geo &, const T *, const T *, const T *, const T *, const T *,      \
                                          T *const[3], T *const[3], StageConst, const TermList[3], const double *,  \
                                          const double *, hipStream_t);                                             \

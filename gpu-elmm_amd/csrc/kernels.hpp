@@ -150,8 +150,8 @@ template <typename T>
 void launch_wm_ustar(const Geo &g, const T *U, const T *V, const T *W, const T *Temp, const T *Moist,
                      WMUstarPoints wp, double nu, T *Visc, hipStream_t st);
 template <typename T>
-void launch_momentum(const Geo &g, int comp, const T *U, const T *V, const T *W, const T *Visc, const T *Pr, T *Ustar,
-                     T *U2, const uint8_t *code, StageConst sc, hipStream_t st);
+void launch_momentum(const Geo &g, const T *U, const T *V, const T *W, const T *Visc, const T *Pr, T *const Us[3],
+                     T *const U2[3], const uint8_t *const code[3], StageConst sc, hipStream_t st);
 // fused three-component momentum kernel, z-marching (k_momentum_zm.hip)
 bool momentum_zm_supported(const Geo &g);
 size_t momentum_zm_lds_bytes(int elem);
