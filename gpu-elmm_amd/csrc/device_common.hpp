@@ -123,6 +123,27 @@ struct StageConst {
   double bA2, bATref;
 };
 
+// Stores v at the interior cell (i, j, k) of a field with one ghost layer and
+// at the ghost cells that take its value (BoundViscosity: periodic x and y,
+// copies of the wall levels in z).
+template <typename T>
+__device__ inline void store_one_layer(const Geo &g, T *__restrict__ F, int i, int j, int k, T v) {
+  auto row = [&](int jj, int kk) {
+    const long p = gix(g, i, jj, kk);
+    F[p] = v;
+    if (i == 1) F[p + g.nx] = v;
+    if (i == g.nx) F[p - g.nx] = v;
+  };
+  auto level = [&](int kk) {
+    row(j, kk);
+    if (j == 1) row(g.ny + 1, kk);
+    if (j == g.ny) row(0, kk);
+  };
+  level(k);
+  if (k == 1) level(0);
+  if (k == g.nz) level(g.nz + 1);
+}
+
 // Ordered per-cell corrections (built on the host in the reference's scatter
 // order).  Cells are listed once; terms[ptr[c]..ptr[c+1]) apply in order.
 struct TermList {

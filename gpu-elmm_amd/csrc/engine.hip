@@ -635,20 +635,20 @@ struct Engine : EngineIface {
     timed(ELMM_T_GHOST, [&] { launch_bound_uvw<T>(g, a, b, c, stream); });
   }
   // BoundUVW after IBMomentum: only the ghost cells whose source is an IB
-  // point change, so only those are rewritten (lists built at set-up;
-  // ELMM_GHOST_DELTA=0 runs the full fill)
+  // point change, so only those are rewritten, with the points' scatter
+  // (lists built at set-up; ELMM_GHOST_DELTA=0 runs the full fill)
   DevBuf gdelta;
   int gdelta_n[3] = {0, 0, 0};
   bool use_gdelta = false;
-  void bound_uvw_after_ib(T *a, T *b, T *c) {
-    if (use_gdelta)
-      timed(ELMM_T_GHOST, [&] { launch_ghost_delta<T>(a, b, c, gdelta.as<long long>(), gdelta_n, stream); });
-    else
-      bound_uvw(a, b, c);
-  }
-  void setup_ghost_delta();
-  void ib_momentum(T *a, T *b, T *c);
-  void pressure_correction(T *a, T *b, T *c, bool use_q, double coef, bool diag = false);
+  // every IB point and every interpolation tap is an interior cell (taps in
+  // ghost cells are replaced by the cells BoundUVW fills them from)
+  bool ib_interior = true;
+  void setup_ghost_delta(const elmm_lists &L);
+  void ib_momentum(T *a, T *b, T *c, bool ghosts);
+  // ghosts: the projection writes the x and y ghost cells of the velocity
+  // and the pressure, launch_bound_z their z layers later; otherwise the
+  // velocity's ghost cells stay as they are and the pressure's are filled
+  void pressure_correction(T *a, T *b, T *c, bool use_q, double coef, bool diag = false, bool ghosts = false);
   void poisson_solve(int accumulate);
   void subgrid_stresses(bool cfl);
   // variable time steps: the first stage's SGS kernel (which also writes the
@@ -1093,10 +1093,10 @@ void Engine<T>::mg_solve() {
 }
 
 template <typename T>
-void Engine<T>::setup_ghost_delta() {
+void Engine<T>::setup_ghost_delta(const elmm_lists &L) {
   use_gdelta = false;
   const char *e = std::getenv("ELMM_GHOST_DELTA");
-  if (!has_ib() || (e && std::string(e) == "0")) return;
+  if (!has_ib() || !ib_interior || (e && std::string(e) == "0")) return;
   long cap = 1;
   for (int c = 0; c < 3; c++) cap = std::max(cap, ghost_shell_cells(g, c));
   DevBuf mark, tmp, cnt;
@@ -1116,6 +1116,18 @@ void Engine<T>::setup_ghost_delta() {
     all.resize(off + 2 * (size_t)n);
     if (n) HIPCHK(hipMemcpy(all.data() + off, tmp.p, 2 * (size_t)n * sizeof(long long), hipMemcpyDeviceToHost));
     gdelta_n[c] = n;
+    // source cells -> IB points (numbered through the three components)
+    std::unordered_map<long long, long long> point;
+    for (int p = 0; p < ib_n[c]; p++) {
+      const int32_t *q = &L.ib_ijk[c][3 * (size_t)p];
+      point[gix(g, q[0], q[1], q[2])] = (c > 0 ? ib_n[0] : 0) + (c > 1 ? ib_n[1] : 0) + p;
+    }
+    const long long neg = 1LL << 62;
+    for (size_t q = off; q < all.size(); q += 2) {
+      const auto it = point.find(all[q + 1] & (neg - 1));
+      if (it == point.end()) throw HipError("ghost delta entry without its point");
+      all[q + 1] = it->second | (all[q + 1] & neg);
+    }
   }
   upload_vec(gdelta, all);
   use_gdelta = true;
@@ -1408,6 +1420,35 @@ void Engine<T>::setup_lists(const elmm_lists &L) {
       int nt = pt.back();
       std::vector<int32_t> sr(L.ib_src_ijk[c], L.ib_src_ijk[c] + 3 * (size_t)nt);
       std::vector<double> cf(L.ib_coef[c], L.ib_coef[c] + nt);
+      if (c < 3) {
+        // taps in ghost cells: the interior cell BoundUVW copies, the sign in
+        // the coefficient (a zero ghost: coefficient 0), so that the
+        // interpolation needs no filled ghost cells
+        auto inside = [&](const int32_t *q) {
+          return q[0] >= 1 && q[0] <= g.n[c][0] && q[1] >= 1 && q[1] <= g.n[c][1] && q[2] >= 1 && q[2] <= g.n[c][2];
+        };
+        std::vector<int32_t> sr2 = sr;
+        std::vector<double> cf2 = cf;
+        bool ok = true;
+        for (int p = 0; p < ib_n[c] && ok; p++) ok = inside(&tg[3 * (size_t)p]);
+        for (int t = 0; t < nt && ok; t++) {
+          int32_t *q = &sr2[3 * (size_t)t];
+          if (inside(q)) continue;
+          int src[3], neg;
+          bool zero;
+          ok = ghost_source(g, c, q[0], q[1], q[2], src, neg, zero);
+          if (zero)
+            q[0] = q[1] = q[2] = 1, cf2[t] = 0;
+          else
+            q[0] = src[0], q[1] = src[1], q[2] = src[2], cf2[t] = neg ? -cf2[t] : cf2[t];
+        }
+        if (ok) {
+          sr = sr2;
+          cf = cf2;
+        } else {
+          ib_interior = false;
+        }
+      }
       if (c == 3 && ib_n[3] > 0) {
         // dependency levels of the sequential ScalFlIBPoints loop
         std::unordered_map<long, int> wlev, rlev;
@@ -1504,12 +1545,29 @@ void Engine<T>::setup_lists(const elmm_lists &L) {
     for (int c = 0; c < 3; c++) {
       null_n[c] = L.null_n[c];
       std::vector<int32_t> v(L.null_ijk[c], L.null_ijk[c] + 3 * (size_t)null_n[c]);
+      // and the x and y ghost cells that hold their images, which the
+      // projection has written by then
+      const int n[2] = {cfg.nx, cfg.ny};
+      for (int p = 0; p < L.null_n[c]; p++) {
+        const int q[3] = {v[3 * (size_t)p], v[3 * (size_t)p + 1], v[3 * (size_t)p + 2]};
+        int im[2][3], ni[2];
+        for (int a = 0; a < 2; a++) {
+          ni[a] = 0;
+          im[a][ni[a]++] = q[a];
+          if (q[a] >= 1 && q[a] <= 3) im[a][ni[a]++] = q[a] + n[a];
+          if (q[a] > n[a] - 3 && q[a] <= n[a]) im[a][ni[a]++] = q[a] - n[a];
+        }
+        for (int b = 0; b < ni[1]; b++)
+          for (int a = 0; a < ni[0]; a++)
+            if (a || b) v.insert(v.end(), {im[0][a], im[1][b], q[2]});
+      }
+      null_n[c] = (int)(v.size() / 3);
       upload_vec(null_ijk[c], v);
     }
   });
   run_parallel(tasks, device);
   tr.mark(" lists");
-  setup_ghost_delta();
+  setup_ghost_delta(L);
   tr.mark(" ghost delta");
 }
 
@@ -1735,9 +1793,11 @@ void Engine<T>::xfer_rows(E *d, const int lo[3], const int hi[3], int lb, const 
 }
 
 template <typename T>
-void Engine<T>::ib_momentum(T *a, T *b, T *c) {
+void Engine<T>::ib_momentum(T *a, T *b, T *c, bool ghosts) {
   const IBDev ib[3] = {ibdev(0), ibdev(1), ibdev(2)};
-  timed(ELMM_T_IB, [&] { launch_ib_momentum(g, ib, a, b, c, ib_tmp.as<double>(), stream); });
+  const long long *list = ghosts && use_gdelta ? gdelta.as<long long>() : nullptr;
+  timed(ELMM_T_IB, [&] { launch_ib_momentum(g, ib, a, b, c, ib_tmp.as<double>(), list, gdelta_n, stream); });
+  if (ghosts && !list) bound_uvw(a, b, c);
 }
 
 template <typename T>
@@ -1779,7 +1839,7 @@ void Engine<T>::poisson_solve(int accumulate) {
 }
 
 template <typename T>
-void Engine<T>::pressure_correction(T *a, T *b, T *c, bool use_q, double coef, bool diag) {
+void Engine<T>::pressure_correction(T *a, T *b, T *c, bool use_q, double coef, bool diag, bool ghosts) {
   const double dt2 = coef, dt2_rec = 1.0 / dt2;
   double *q = use_q ? Q.as<double>() : nullptr;
   const uint32_t *qm = use_q ? qmask.as<uint32_t>() : nullptr;
@@ -1803,9 +1863,9 @@ void Engine<T>::pressure_correction(T *a, T *b, T *c, bool use_q, double coef, b
       launch_top_sum(g, Pr.as<T>(), Phi.as<double>(), partial.as<double>(), top_blocks, stream);
     });
     timed(ELMM_T_PROJECTION, [&] {
-      launch_projection(g, a, b, c, Pr.as<T>(), Phi.as<double>(), partial.as<double>(), top_blocks, dt2, stream);
+      launch_projection(g, a, b, c, Pr.as<T>(), Phi.as<double>(), partial.as<double>(), top_blocks, dt2, ghosts, stream);
     });
-    timed(ELMM_T_GHOST, [&] { launch_bound_pr<T>(g, Pr.as<T>(), stream); });
+    if (!ghosts) timed(ELMM_T_GHOST, [&] { launch_bound_pr<T>(g, Pr.as<T>(), stream); });
     return;
   }
   timed(ELMM_T_POISSON_X_FWD, [&] {
@@ -1836,9 +1896,9 @@ void Engine<T>::pressure_correction(T *a, T *b, T *c, bool use_q, double coef, b
     launch_top_sum(g, Pr.as<T>(), Phi.as<double>(), partial.as<double>(), top_blocks, stream);
   });
   timed(ELMM_T_PROJECTION, [&] {
-    launch_projection(g, a, b, c, Pr.as<T>(), Phi.as<double>(), partial.as<double>(), top_blocks, dt2, stream);
+    launch_projection(g, a, b, c, Pr.as<T>(), Phi.as<double>(), partial.as<double>(), top_blocks, dt2, ghosts, stream);
   });
-  timed(ELMM_T_GHOST, [&] { launch_bound_pr<T>(g, Pr.as<T>(), stream); });
+  if (!ghosts) timed(ELMM_T_GHOST, [&] { launch_bound_pr<T>(g, Pr.as<T>(), stream); });
 }
 
 // SubgridStresses, src/dynamics.f90:869-908 (ComputeViscsWM only writes
@@ -1859,12 +1919,15 @@ void Engine<T>::subgrid_stresses(bool cfl) {
   // constant dt with the CFL check: the step's CFL number and the divergence
   // test, on the device (graph-safe)
   if (cfl && !cfg.variable_dt)
-    timed(ELMM_T_REDUCE, [&] {
-      launch_cfl_monitor(cfl_partial.as<double>(), cfl_blocks, dt_cur, cfg.cfl_max, mon, stream);
-    });
-  if (cfg.wall_model && wm_n)
-    timed(ELMM_T_WALL, [&] { launch_wm_fluxes(g, u, v, w, temp_cur(), moist_cur(), wmdev(), cfg.nu, g.variable_z, stream); });
-  timed(ELMM_T_GHOST, [&] { launch_bound_visc<T>(g, Visc.as<T>(), stream); });
+    sw.cfl = CflArgs{cfl_partial.as<double>(), cfl_blocks, dt_cur, cfg.cfl_max, mon};
+  sw.wm = wmdev();
+  sw.wp = wmpdev();
+  sw.div = WMScalarPoints{nsc > 0 ? wmp_n : 0, wmp_ijk.as<int32_t>(), wmp_div.as<double>()};
+  if (!cfg.wall_model) sw.wm.n = sw.wp.n = 0;
+  sw.prtype = prtype.as<int32_t>();
+  sw.visc = Visc.as<T>();
+  sw.nu = cfg.nu;
+  timed(ELMM_T_WALL, [&] { launch_surface<T>(g, u, v, w, temp_cur(), moist_cur(), sw, stream); });
   if (ib_n[3])
     timed(ELMM_T_IB, [&] {
       launch_ib_visc_serial(g, ibdev(3), Visc.as<T>(), visc_levels.data(), (int)visc_levels.size() - 1, stream);
@@ -1872,10 +1935,8 @@ void Engine<T>::subgrid_stresses(bool cfl) {
   // ComputeTDiff (src/scalar_diffusion.f90:983-1009) with buoyancy, then
   // BoundViscosity(TDiff); without it TDiff keeps its initial values
   if (cfg.enable_buoyancy)
-    timed(ELMM_T_OTHER, [&] {
-      launch_tdiff_init(g, Visc.as<T>(), TDiff.as<T>(), cfg.nu, cfg.nu_scalar, stream);
-      launch_bound_visc<T>(g, TDiff.as<T>(), stream);
-    });
+    timed(ELMM_T_OTHER,
+          [&] { launch_tdiff_init(g, Visc.as<T>(), TDiff.as<T>(), cfg.nu, cfg.nu_scalar, stream); });
 }
 
 template <typename T>
@@ -1967,14 +2028,15 @@ void Engine<T>::stage(int st, bool last) {
       std::swap(s_cur[s], s_nxt[s]);
     }
   }
-  bound_uvw(u2, v2, w2);
+  // BoundUVW of the new velocity: nothing before the projection reads its
+  // ghost cells (the divergence wraps its indices, IB taps are interior)
   const bool use_q = cfg.ib_mass_sources && has_ib();
   if (has_ib()) {
-    ib_momentum(u2, v2, w2);
-    bound_uvw_after_ib(u2, v2, w2);
+    if (!ib_interior) bound_uvw(u2, v2, w2);
+    ib_momentum(u2, v2, w2, false);
   }
   if (use_q) timed(ELMM_T_IB, [&] { launch_mass_sources(g, q_terms.view(), u2, v2, w2, Q.as<double>(), stream); });
-  pressure_correction(u2, v2, w2, use_q, sc.coef, last && want_diag);
+  pressure_correction(u2, v2, w2, use_q, sc.coef, last && want_diag, true);
   if (cfg.delta_diag)
     timed(ELMM_T_REDUCE, [&] {
       launch_delta<T>(g, u, u2, v, v2, w, w2, delta_partial.as<double>(), dblocks, st, dt, mon, stream);
@@ -1991,11 +2053,8 @@ void Engine<T>::stage(int st, bool last) {
     const int32_t *const nl[3] = {null_ijk[0].as<int32_t>(), null_ijk[1].as<int32_t>(), null_ijk[2].as<int32_t>()};
     timed(ELMM_T_IB, [&] { launch_null(g, null_n, nl, u, v, w, stream); });
   }
-  bound_uvw(u, v, w);
-  if (has_ib()) {
-    ib_momentum(u, v, w);
-    bound_uvw_after_ib(u, v, w);
-  }
+  timed(ELMM_T_GHOST, [&] { launch_bound_z<T>(g, u, v, w, Pr.as<T>(), stream); });
+  if (has_ib()) ib_momentum(u, v, w, true);
 }
 
 template <typename T>
@@ -2010,10 +2069,7 @@ void Engine<T>::init() {
   launch_sgs(g, u, v, w, Visc.as<T>(), cfg.nu, cfg.c_smag, cfg.filter_ratio,
              sgs_width, cfg.sgs_model, nullptr, 0, stream);
   launch_bound_visc<T>(g, Visc.as<T>(), stream);
-  if (nsc > 0) {
-    launch_tdiff_init(g, Visc.as<T>(), TDiff.as<T>(), cfg.nu, cfg.nu_scalar, stream);
-    launch_bound_visc<T>(g, TDiff.as<T>(), stream);
-  }
+  if (nsc > 0) launch_tdiff_init(g, Visc.as<T>(), TDiff.as<T>(), cfg.nu, cfg.nu_scalar, stream);
   for (int s = 0; s < nsc; s++) launch_bound_scalar<T>(gscal(s), s_cur[s], stream);
   if (cfg.wall_model && wmp_n) launch_wm_ustar<T>(g, u, v, w, temp_cur(), moist_cur(), wmpdev(), cfg.nu, Visc.as<T>(), stream);
   if (cfg.wall_model) launch_wm_fluxes(g, u, v, w, temp_cur(), moist_cur(), wmdev(), cfg.nu, g.variable_z, stream);
@@ -2029,7 +2085,7 @@ template <typename T>
 void Engine<T>::first_call() {
   if (first_step_done) return;
   bound_uvw(u, v, w);
-  if (has_ib()) ib_momentum(u, v, w);
+  if (has_ib()) ib_momentum(u, v, w, false);
   first_step_done = true;
 }
 

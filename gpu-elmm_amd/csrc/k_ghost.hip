@@ -79,7 +79,7 @@ __device__ inline bool decode(const Shell &s, long t_, int &i, int &j, int &k) {
 // ---------------------------------------------------------------- BoundUVW
 // Per-axis velocity rule (src/boundaries.f90:461-572, 783-894, 1122-1233,
 // 1323-1434, 1533-1647, 1676-1789). Returns true for a zero value.
-__device__ inline bool vel_rule(int m, int n, int blo, int bhi, bool normal, int &src, int &neg) {
+__host__ __device__ inline bool vel_rule(int m, int n, int blo, int bhi, bool normal, int &src, int &neg) {
   if (m <= 0) {
     if (blo == BCN_PERIODIC) { src = m + n; neg = 0; return false; }
     if (normal) {
@@ -166,17 +166,41 @@ __global__ void k_mark_cells(Geo g, const int32_t *__restrict__ ijk, int n, uint
   if (p < n) mark[gix(g, ijk[3 * p], ijk[3 * p + 1], ijk[3 * p + 2])] = v;
 }
 
-// Re-applies the listed ghost rules (n[c] entries per component, U's
-// first): after a change of the listed source cells only, this equals a full
-// BoundUVW.
+// The z ghost layers of the three velocity components and of the pressure
+// (blockIdx.y = 3; Bound_Pr's extrapolation on the interior columns), from
+// fields whose x and y ghost cells hold their values already: with the outer
+// rule applied last, this completes BoundUVW and Bound_Pr.
 template <typename T>
-__global__ void k_ghost_delta(T *U, T *V, T *W, const long long *__restrict__ list, int n0, int n1, int n2) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n0 + n1 + n2) return;
-  T *F = q < n0 ? U : q < n0 + n1 ? V : W;
-  const long long dst = list[2 * q], e = list[2 * q + 1];
-  const T v = F[e & ((1LL << 62) - 1)];
-  F[dst] = (e >> 62) ? -v : v;
+__global__ void k_bound_z(Geo g, T *U, T *V, T *W, T *P) {
+  const int c = blockIdx.y;
+  const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c < 3) {
+    T *F = c == 0 ? U : c == 1 ? V : W;
+    const unsigned w = (unsigned)g.nx + 6, h = (unsigned)g.ny + 6, r = t / w, l = r / h;
+    if (l >= 6) return;
+    const int i = (int)(t - r * w) - 2, j = (int)(r - l * h) - 2, n = g.n[c][2];
+    const int k = ghost_index((int)l, 3, n);
+    int sk = 1, neg = 0;
+    const bool zero = vel_rule(k, n, g.bt[4], g.bt[5], c == 2, sk, neg);
+    const T src = F[gix(g, i, j, zero ? 1 : sk)];
+    const T v = zero ? T(0) : src;
+    F[gix(g, i, j, k)] = !zero && neg ? -v : v;
+  } else {
+    const unsigned w = (unsigned)g.nx, h = (unsigned)g.ny, r = t / w, l = r / h;
+    if (l >= 2) return;
+    const long p = gix(g, (int)(t - r * w) + 1, (int)(r - l * h) + 1, 0);
+    const int n = g.nz;
+    auto at = [&](int k) -> T & { return P[p + (long)k * g.sz]; };
+    if (l == 0) {
+      const T p1 = at(1), p2 = at(2), p3 = at(3);
+      at(0) = p3 - 3 * (p2 - p1);
+      at(-1) = p2;
+    } else {
+      const T p0 = at(n), p1 = at(n - 1), p2 = at(n - 2);
+      at(n + 1) = p2 - 3 * (p1 - p0);
+      at(n + 2) = p1;
+    }
+  }
 }
 
 // ------------------------------------------------------ BoundViscosity
@@ -324,6 +348,26 @@ void launch_bound_uvw(const Geo &g, T *U, T *V, T *W, hipStream_t st) {
   hipLaunchKernelGGL(k_bound_uvw<T>, dim3(nblk(mx, 256), 3), dim3(256), 0, st, g, U, V, W, s[0], s[1], s[2]);
 }
 
+template <typename T>
+void launch_bound_z(const Geo &g, T *U, T *V, T *W, T *P, hipStream_t st) {
+  const long n = 6L * (g.nx + 6) * (g.ny + 6);
+  hipLaunchKernelGGL(k_bound_z<T>, dim3(nblk(n, 256), 4), dim3(256), 0, st, g, U, V, W, P);
+}
+
+bool ghost_source(const Geo &g, int c, int i, int j, int k, int src[3], int &neg, bool &zero) {
+  const int n[3] = {g.n[c][0], g.n[c][1], g.n[c][2]}, q[3] = {i, j, k};
+  neg = 0;
+  zero = false;
+  for (int a = 2; a >= 0; a--) {
+    src[a] = q[a];
+    if (zero || (q[a] >= 1 && q[a] <= n[a])) continue;
+    int nn = 0;
+    zero = vel_rule(q[a], n[a], g.bt[2 * a], g.bt[2 * a + 1], a == c, src[a], nn);
+    if (!zero) neg ^= nn;
+  }
+  return zero || (src[0] >= 1 && src[0] <= n[0] && src[1] >= 1 && src[1] <= n[1] && src[2] >= 1 && src[2] <= n[2]);
+}
+
 long ghost_shell_cells(const Geo &g, int c) {
   const Shell s = uvw_shell(g, c);
   return s.cz + s.cy + s.cx;
@@ -344,12 +388,6 @@ int ghost_delta_build(const Geo &g, int c, const int32_t *ijk, int n, uint8_t *m
 }
 
 template <typename T>
-void launch_ghost_delta(T *U, T *V, T *W, const long long *list, const int n[3], hipStream_t st) {
-  const int tot = n[0] + n[1] + n[2];
-  if (tot) hipLaunchKernelGGL(k_ghost_delta<T>, dim3(nblk(tot, 256)), dim3(256), 0, st, U, V, W, list, n[0], n[1], n[2]);
-}
-
-template <typename T>
 void launch_bound_visc(const Geo &g, T *F, hipStream_t st) {
   Shell s = make_shell(g.nx, g.ny, g.nz, 1, 1, 0, g.nx + 1, 0, g.ny + 1, 0, g.nx + 1);
   hipLaunchKernelGGL(k_bound_visc<T>, dim3(nblk(s.cz + s.cy + s.cx, 256)), dim3(256), 0, st, g, F, s);
@@ -367,10 +405,10 @@ void launch_bound_pr(const Geo &g, T *P, hipStream_t st) {
   hipLaunchKernelGGL(k_bound_pr<T>, dim3(nblk(s.cz + s.cy + s.cx, 256)), dim3(256), 0, st, g, P, s);
 }
 
-template void launch_ghost_delta<double>(double *, double *, double *, const long long *, const int[3], hipStream_t);
-template void launch_ghost_delta<float>(float *, float *, float *, const long long *, const int[3], hipStream_t);
 template void launch_bound_uvw<double>(const Geo &, double *, double *, double *, hipStream_t);
 template void launch_bound_uvw<float>(const Geo &, float *, float *, float *, hipStream_t);
+template void launch_bound_z<double>(const Geo &, double *, double *, double *, double *, hipStream_t);
+template void launch_bound_z<float>(const Geo &, float *, float *, float *, float *, hipStream_t);
 template void launch_bound_visc<double>(const Geo &, double *, hipStream_t);
 template void launch_bound_visc<float>(const Geo &, float *, hipStream_t);
 template void launch_bound_scalar<double>(const Geo &, double *, hipStream_t);

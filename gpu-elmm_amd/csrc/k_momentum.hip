@@ -777,6 +777,149 @@ __global__ void k_wm_ustar(Geo g, const T *__restrict__ U_, const T *__restrict_
         visc = nu;
     }
   }
+template <typename T>
+__global__ void k_wm_ustar(Geo g, const T *__restrict__ U, const T *__restrict__ V, const T *__restrict__ W,
+                           const T *__restrict__ Temp, const T *__restrict__ Moist, WMUstarPoints wp, double nu,
+                           T *__restrict__ Visc) {
+  wm_ustar_point<T>(g, U, V, W, Temp, Moist, wp, nu, Visc, blockIdx.x * blockDim.x + threadIdx.x);
+}
+template <typename T>
+__global__ void k_wm_fluxes(Geo g, const T *__restrict__ U, const T *__restrict__ V, const T *__restrict__ W,
+                            const T *__restrict__ Temp, const T *__restrict__ Moist, WMPoints wm, double nu,
+                            int variable_z) {
+  wm_flux_point<T>(g, U, V, W, Temp, Moist, wm, nu, variable_z, blockIdx.x * blockDim.x + threadIdx.x);
+}
+
+template <typename T>
+void launch_wm_fluxes(const Geo &g, const T *U, const T *V, const T *W, const T *Temp, const T *Moist, WMPoints wm,
+                      double nu, int variable_z, hipStream_t st) {
+  if (wm.n == 0) return;
+  hipLaunchKernelGGL(k_wm_fluxes<T>, dim3(nblk(wm.n, 256)), dim3(256), 0, st, g, U, V, W, Temp, Moist, wm, nu,
+                     variable_z);
+}
+
+// DivergenceWM (2nd order), src/wallmodels.f90:1153-1166
+template <typename Real>
+__device__ inline void wm_div_point(const Geo &g, const WMScalarPoints &wp, const int32_t *__restrict__ pt,
+                                    const Real *__restrict__ U_, const Real *__restrict__ V_,
+                                    const Real *__restrict__ W_, int n) {
+  if (n >= wp.n) return;
+  auto U = [&](long q) { return (double)U_[q]; };
+  auto V = [&](long q) { return (double)V_[q]; };
+  auto W = [&](long q) { return (double)W_[q]; };
+  const int xi = wp.ijk[3 * n], yj = wp.ijk[3 * n + 1], zk = wp.ijk[3 * n + 2];
+  const long p = gix(g, xi, yj, zk);
+  const long sy = g.sy, sz = g.sz;
+  double div = 0;
+  if (pt[p + 1] <= 0) div = div + U(p) / g.dxmin;
+  if (pt[p - 1] <= 0) div = div - U(p - 1) / g.dxmin;
+  if (pt[p + sy] <= 0) div = div + V(p) / g.dymin;
+  if (pt[p - sy] <= 0) div = div - V(p - sy) / g.dymin;
+  if (pt[p + sz] <= 0) div = div + W(p) / g.dzPr[zk];
+  if (pt[p - sz] <= 0) div = div - W(p - sz) / g.dzPr[zk];
+  wp.div[n] = div;
+}
+
+// Ghost cell t of the viscosity's one layer (BoundViscosity: x, then y over
+// the x ghosts, then z over both; periodic x and y, copies in z).
+template <typename T>
+__device__ inline void visc_ghost(const Geo &g, T *__restrict__ F, unsigned t) {
+  const unsigned wx = (unsigned)g.nx + 2, wy = (unsigned)g.ny + 2, cz = 2 * wx * wy, cy = 2 * wx * (unsigned)g.nz;
+  int i, j, k;
+  if (t < cz) {
+    const unsigned r = t / wx, l = r / wy;
+    i = (int)(t - r * wx);
+    j = (int)(r - l * wy);
+    k = l ? g.nz + 1 : 0;
+  } else if ((t -= cz) < cy) {
+    const unsigned r = t / wx;
+    i = (int)(t - r * wx);
+    j = r & 1 ? g.ny + 1 : 0;
+    k = 1 + (int)(r >> 1);
+  } else {
+    t -= cy;
+    const unsigned r = t >> 1, l = r / (unsigned)g.ny;
+    if (l >= (unsigned)g.nz) return;
+    i = t & 1 ? g.nx + 1 : 0;
+    j = 1 + (int)(r - l * (unsigned)g.ny);
+    k = 1 + (int)l;
+  }
+  const int si = i == 0 ? g.nx : i == g.nx + 1 ? 1 : i, sj = j == 0 ? g.ny : j == g.ny + 1 ? 1 : j;
+  const int sk = k == 0 ? 1 : k == g.nz + 1 ? g.nz : k;
+  F[gix(g, i, j, k)] = F[gix(g, si, sj, sk)];
+}
+
+// TimeStepLength's maximum (src/dynamics.f90:556-591) from the block maxima
+// the SGS kernel wrote at the first stage, then main.f90's divergence test
+// (src/main.f90:161-168: time_step >= 3, CFL > CFL_max; a NaN velocity makes
+// the maximum huge, src/dynamics.f90:538).  One block of 256 threads.
+__device__ inline void cfl_monitor(const CflArgs &a) {
+  auto nan_max = [](double x, double y) { return x != x || y != y ? (double)INFINITY : x > y ? x : y; };
+  double v = 0;
+  for (int b = threadIdx.x; b < a.nblocks; b += 256) v = nan_max(v, a.partial[b]);
+  for (int off = 32; off > 0; off >>= 1) v = nan_max(v, __shfl_xor(v, off));
+  __shared__ double red[4];
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  double m = red[0];
+  for (int w = 1; w < 4; w++) m = nan_max(m, red[w]);
+  const double cfl = m * a.dt;
+  StepMon *mon = a.mon;
+  const long long step = mon->step + 1;
+  mon->step = step;
+  mon->cfl_last = cfl;
+  mon->umax_last = m;
+  if (a.cfl_max > 0 && step >= 3 && !(cfl <= a.cfl_max) && mon->first_bad < 0) mon->first_bad = step;
+}
+
+// The stage-start work on lists and surfaces, which only reads the velocity
+// (and the viscosity's interior) and writes arrays of its own: the CFL
+// monitor, the wall fluxes of the momentum points, u* and the divergence of
+// the scalar wall-model points and the viscosity's ghost layer, each in
+// blocks of its own of one launch.  Apart they take 4.7 us each on small
+// grids (a launch and a memory round trip or two) and run one after another
+// with most of the chip idle (urban 512x512x128: 37 + 17 + 11 + 14 us).
+template <typename T>
+__global__ void __launch_bounds__(256)
+    k_surface(Geo g, const T *__restrict__ U, const T *__restrict__ V, const T *__restrict__ W,
+              const T *__restrict__ Temp, const T *__restrict__ Moist, SurfaceWork<T> s) {
+  int b = blockIdx.x;
+  if (b < s.b_cfl) {
+    cfl_monitor(s.cfl);
+    return;
+  }
+  b -= s.b_cfl;
+  if (b < s.b_flux) {
+    wm_flux_point<T>(g, U, V, W, Temp, Moist, s.wm, s.nu, g.variable_z, b * 256 + threadIdx.x);
+    return;
+  }
+  b -= s.b_flux;
+  if (b < s.b_ustar) {
+    wm_ustar_point<T>(g, U, V, W, Temp, Moist, s.wp, s.nu, (T *)nullptr, b * 256 + threadIdx.x);
+    return;
+  }
+  b -= s.b_ustar;
+  if (b < s.b_div) {
+    wm_div_point<T>(g, s.div, s.prtype, U, V, W, b * 256 + threadIdx.x);
+    return;
+  }
+  b -= s.b_div;
+  visc_ghost<T>(g, s.visc, (unsigned)b * 256u + threadIdx.x);
+}
+
+template <typename T>
+void launch_surface(const Geo &g, const T *U, const T *V, const T *W, const T *Temp, const T *Moist,
+                    SurfaceWork<T> s, hipStream_t st) {
+  s.b_cfl = s.cfl.mon ? 1 : 0;
+  s.b_flux = (int)nblk(s.wm.n, 256);
+  s.b_ustar = (int)nblk(s.wp.n, 256);
+  s.b_div = (int)nblk(s.div.n, 256);
+  const long ghosts = 2L * (g.nx + 2) * (g.ny + 2) + 2L * (g.nx + 2) * g.nz + 2L * g.ny * g.nz;
+  hipLaunchKernelGGL(k_surface<T>, dim3(s.b_cfl + s.b_flux + s.b_ustar + s.b_div + nblk(ghosts, 256)), dim3(256), 0, st,
+                     g, U, V, W, Temp, Moist, s);
+}
+
   wp.ustar[p] = ustar;
   if (Visc) Visc[q] = (T)visc;
   // TemperatureExtra's surface source (src/scalars.f90:322-326)
@@ -1230,20 +1373,31 @@ __global__ void k_ib_interp(Geo g, IB3 ib, const T *__restrict__ U, const T *__r
   tmp[p] = s;
 }
 template <typename T>
-__global__ void k_ib_scatter(Geo g, IB3 ib, const double *__restrict__ tmp, T *__restrict__ U, T *__restrict__ V,
-                             T *__restrict__ W) {
+__global__ void k_ib_scatter(Geo g, IB3 ib, const double *__restrict__ tmp, const long long *__restrict__ ghosts,
+                             int g0, int g01, int g012, T *__restrict__ U, T *__restrict__ V, T *__restrict__ W) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= ib.n012) return;
+  if (p >= ib.n012) {
+    const int q = p - ib.n012;
+    if (q >= g012) return;
+    T *F = q < g0 ? U : q < g01 ? V : W;
+    const long long e = ghosts[2 * q + 1];
+    const T v = (T)tmp[e & ((1LL << 62) - 1)];
+    F[ghosts[2 * q]] = (e >> 62) ? -v : v;
+    return;
+  }
   const IBSel d = ib_pick(ib, p);
   T *F = p < ib.n0 ? U : p < ib.n01 ? V : W;
   F[gix(g, d.tgt[3 * d.q], d.tgt[3 * d.q + 1], d.tgt[3 * d.q + 2])] = (T)tmp[p];
 }
 template <typename T>
-void launch_ib_momentum(const Geo &g, const IBDev ib[3], T *U, T *V, T *W, double *tmp, hipStream_t st) {
+void launch_ib_momentum(const Geo &g, const IBDev ib[3], T *U, T *V, T *W, double *tmp, const long long *ghosts,
+                        const int nghost[3], hipStream_t st) {
   IB3 b{ib[0], ib[1], ib[2], ib[0].n, ib[0].n + ib[1].n, ib[0].n + ib[1].n + ib[2].n};
   if (!b.n012) return;
   hipLaunchKernelGGL(k_ib_interp<T>, dim3(nblk(b.n012, 256)), dim3(256), 0, st, g, b, U, V, W, tmp);
-  hipLaunchKernelGGL(k_ib_scatter<T>, dim3(nblk(b.n012, 256)), dim3(256), 0, st, g, b, tmp, U, V, W);
+  const int g0 = ghosts ? nghost[0] : 0, g01 = ghosts ? g0 + nghost[1] : 0, g012 = ghosts ? g01 + nghost[2] : 0;
+  hipLaunchKernelGGL(k_ib_scatter<T>, dim3(nblk((long)b.n012 + g012, 256)), dim3(256), 0, st, g, b, tmp, ghosts, g0,
+                     g01, g012, U, V, W);
 }
 
 // ScalFlIBPoints viscosity loop (src/dynamics.f90:899-902) is sequential:
@@ -1394,7 +1548,8 @@ void launch_mass_sources(const Geo &g, TermList tl, const T *U, const T *V, cons
   template void launch_momentum_corr<T>(const Geo &, int, const T *, const T *, const T *, const T *, const T *,   \
                                         T *, T *, const uint8_t *, StageConst, TermList, const double *,           \
                                         const double *, hipStream_t);                                              \
-  template void launch_ib_momentum<T>(const Geo &, const IBDev[3], T *, T *, T *, double *, hipStream_t);         \
+  template void launch_ib_momentum<T>(const Geo &, const IBDev[3], T *, T *, T *, double *, const long long *,      \
+                                      const int[3], hipStream_t);         \
   template void launch_ib_visc_serial<T>(const Geo &, IBDev, T *, const int32_t *, int, hipStream_t);              \
   template void launch_null<T>(const Geo &, const int[3], const int32_t *const[3], T *, T *, T *, hipStream_t);    \
   template void launch_mass_sources<T>(const Geo &, TermList, const T *, const T *, const T *, double *,           \

@@ -66,7 +66,9 @@ __global__ void __launch_bounds__(256) k_mg_rhs(Geo g, const T *__restrict__ U, 
   const int i = (int)(t % g.nx) + 1, j = (int)((t / g.nx) % g.ny) + 1, k = (int)(t / ((long)g.nx * g.ny)) + 1;
   const long p = gix(g, i, j, k);
   const double dz = g.variable_z ? g.dzPr[k] : g.dzmin;
-  double r = ((double)U[p] - (double)U[p - 1]) / g.dxmin + ((double)V[p] - (double)V[p - g.sy]) / g.dymin +
+  // U(0) and V(0) by index wrap (periodic x and y)
+  const long pw = i > 1 ? p - 1 : p - 1 + g.nx, ps = j > 1 ? p - g.sy : p - g.sy + (long)g.ny * g.sy;
+  double r = ((double)U[p] - (double)U[pw]) / g.dxmin + ((double)V[p] - (double)V[ps]) / g.dymin +
              ((double)W[p] - (double)W[p - g.sz]) / dz;
   if (Q) r = r - Q[p];
   r = r * dt2_rec;

@@ -224,7 +224,11 @@ __global__ void __launch_bounds__(kFftThreads)
     } else if constexpr (MODE == kRhsIn) {
       return rhs_in[p];
     } else {
-      const double du = (double)U[p] - (double)U[p - 1], dv = (double)V[p] - (double)V[p - g.sy];
+      // U(0) and V(0) by index wrap (periodic x and y): the ghost cells of the
+      // stage's velocity are filled after the projection only; W(0) = 0 of
+      // the wall is in the field
+      const double du = (double)U[p] - (double)U[m > 0 ? p - 1 : p - 1 + g.nx];
+      const double dv = (double)V[p] - (double)V[(row & (pp.ny - 1)) > 0 ? p - g.sy : p - g.sy + (long)g.ny * g.sy];
       const double dw = (double)W[p] - (double)W[p - g.sz];
       if constexpr ((MODE & kRhsFast) != 0)
         return div_rn_nz(du, g.dxmin, g.rdx) + div_rn_nz(dv, g.dymin, g.rdy) + div_rn_nz(dw, g.dzmin, g.rdz);
@@ -909,7 +913,12 @@ void launch_top_sum(const Geo &g, const T *Pr, const double *Phi, double *partia
 // U -= coef*(Phi(i+1)-Phi(i))/dx etc. (src/pressure.f90:789-853).  x and y
 // are periodic, so Phi(nx+1) = Phi(1) is read by index wrap (Bound_Phi).
 // The correction is evaluated in FP64 and rounded to the field type T.
-template <typename T>
+// With GHOSTS the kernel also writes the x and y ghost cells that take the
+// values it has in registers (BoundUVW's three layers with their corners,
+// Bound_Pr's two on the faces; periodic, at least 4 cells a direction), whose
+// lines a separate fill would read and write again (three launches and 75 us
+// of a stage on 512x512x128); the z layers follow in launch_bound_z.
+template <typename T, bool GHOSTS>
 __global__ void __launch_bounds__(256)
     k_projection(Geo g, T *__restrict__ U, T *__restrict__ V, T *__restrict__ W, T *__restrict__ Pr,
                  const double *__restrict__ Phi, const double *__restrict__ partial, int nblocks, double dt2) {
@@ -928,24 +937,48 @@ __global__ void __launch_bounds__(256)
   const double phz = Phi[p + g.sz];
   const T u = U[p], v = V[p], w = W[p], pr0 = Pr[p];
   const double Au = dt2 / g.dxmin, Av = dt2 / g.dymin, Aw = dt2 / g.dzmin;
-  if (i <= g.n[0][0] && j <= g.n[0][1] && k <= g.n[0][2]) U[p] = (T)((double)u - Au * (phx - ph));
-  if (i <= g.n[1][0] && j <= g.n[1][1] && k <= g.n[1][2]) V[p] = (T)((double)v - Av * (phy - ph));
-  if (i <= g.n[2][0] && j <= g.n[2][1] && k <= g.n[2][2]) {
+  const long ty = (long)g.ny * g.sy;
+  auto row = [&](T *__restrict__ F, long q, T x) {
+    F[q] = x;
+    if constexpr (GHOSTS) {
+      if (i <= 3) F[q + g.nx] = x;
+      if (i > g.nx - 3) F[q - g.nx] = x;
+    }
+  };
+  auto put = [&](T *__restrict__ F, T x) {
+    row(F, p, x);
+    if constexpr (GHOSTS) {
+      if (j <= 3) row(F, p + ty, x);
+      if (j > g.ny - 3) row(F, p - ty, x);
+    }
+  };
+  put(U, (T)((double)u - Au * (phx - ph)));
+  put(V, (T)((double)v - Av * (phy - ph)));
+  if (k <= g.n[2][2]) {
     if (g.variable_z)
-      W[p] = (T)((double)w - dt2 * (phz - ph) / g.dzW[k]);
+      put(W, (T)((double)w - dt2 * (phz - ph) / g.dzW[k]));
     else
-      W[p] = (T)((double)w - Aw * (phz - ph));
+      put(W, (T)((double)w - Aw * (phz - ph)));
   }
   double pr = (double)pr0 + ph;
   if (ref != 0) pr = pr - ref;
   Pr[p] = (T)pr;
+  if constexpr (GHOSTS) {
+    if (i <= 2) Pr[p + g.nx] = (T)pr;
+    if (i > g.nx - 2) Pr[p - g.nx] = (T)pr;
+    if (j <= 2) Pr[p + ty] = (T)pr;
+    if (j > g.ny - 2) Pr[p - ty] = (T)pr;
+  }
 }
 
 template <typename T>
 void launch_projection(const Geo &g, T *U, T *V, T *W, T *Pr, const double *Phi, const double *partial, int nblocks,
-                       double dt2, hipStream_t st) {
+                       double dt2, bool ghosts, hipStream_t st) {
   dim3 b(64, 4, 1), gr(nblk(g.nx, 64), nblk(g.ny, 4), g.nz);
-  hipLaunchKernelGGL(k_projection<T>, gr, b, 0, st, g, U, V, W, Pr, Phi, partial, nblocks, dt2);
+  if (ghosts)
+    hipLaunchKernelGGL((k_projection<T, true>), gr, b, 0, st, g, U, V, W, Pr, Phi, partial, nblocks, dt2);
+  else
+    hipLaunchKernelGGL((k_projection<T, false>), gr, b, 0, st, g, U, V, W, Pr, Phi, partial, nblocks, dt2);
 }
 
 // max |div U - Q| (check_divergence, src/pressure.f90:937-981)
@@ -1054,7 +1087,7 @@ void launch_refine_residual(const Geo &g, const double *Phi, const double *RHS, 
 #define ELMM_INST_PRESSURE_T(T)                                                                                    \
   template void launch_top_sum<T>(const Geo &, const T *, const double *, double *, int, hipStream_t);             \
   template void launch_projection<T>(const Geo &, T *, T *, T *, T *, const double *, const double *, int, double,  \
-                                     hipStream_t);                                                                 \
+                                     bool, hipStream_t);                                                           \
   template void launch_max_div<T>(const Geo &, const T *, const T *, const T *, const double *, double *, int,      \
                                   hipStream_t);
 ELMM_INST_PRESSURE_R(double)

@@ -407,36 +407,8 @@ void launch_scalar_corr(const Geo &g, const Real *U, const Real *V, const Real *
                      mx, my, mz, sc, tl, src_flux, wm_div);
 }
 
-// DivergenceWM (2nd order), src/wallmodels.f90:1153-1166
-template <typename Real>
-__global__ void k_wm_div(Geo g, WMScalarPoints wp, const int32_t *__restrict__ pt, const Real *__restrict__ U_,
-                         const Real *__restrict__ V_, const Real *__restrict__ W_) {
-  auto U = [&](long q) { return (double)U_[q]; };
-  auto V = [&](long q) { return (double)V_[q]; };
-  auto W = [&](long q) { return (double)W_[q]; };
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= wp.n) return;
-  const int xi = wp.ijk[3 * n], yj = wp.ijk[3 * n + 1], zk = wp.ijk[3 * n + 2];
-  const long p = gix(g, xi, yj, zk);
-  const long sy = g.sy, sz = g.sz;
-  double div = 0;
-  if (pt[p + 1] <= 0) div = div + U(p) / g.dxmin;
-  if (pt[p - 1] <= 0) div = div - U(p - 1) / g.dxmin;
-  if (pt[p + sy] <= 0) div = div + V(p) / g.dymin;
-  if (pt[p - sy] <= 0) div = div - V(p - sy) / g.dymin;
-  if (pt[p + sz] <= 0) div = div + W(p) / g.dzPr[zk];
-  if (pt[p - sz] <= 0) div = div - W(p - sz) / g.dzPr[zk];
-  wp.div[n] = div;
-}
-
-template <typename Real>
-void launch_wm_div(const Geo &g, WMScalarPoints p, const int32_t *prtype, const Real *U, const Real *V, const Real *W,
-                   hipStream_t st) {
-  if (p.n) hipLaunchKernelGGL(k_wm_div<Real>, dim3(nblk(p.n, 256)), dim3(256), 0, st, g, p, prtype, U, V, W);
-}
-
-// TDiff = (Viscosity - molecular_viscosity)/constPr_sgs + molecular_diffusivity,
-// src/initial.f90:4302-4313 (constPr_sgs = 0.6 as a default-real literal)
+// TDiff = (Viscosity - molecular_viscosity)/constPr_sgs + molecular_diffusivity
+// and its ghost layer (BoundViscosity), src/initial.f90:4302-4313 (constPr_sgs = 0.6 as a default-real literal)
 template <typename Real>
 __global__ void k_tdiff_init(Geo g, const Real *__restrict__ Visc, Real *__restrict__ TDiff, double nu,
                              double nu_scalar) {
@@ -445,7 +417,7 @@ __global__ void k_tdiff_init(Geo g, const Real *__restrict__ Visc, Real *__restr
   const int k = blockIdx.z + 1;
   if (i > g.nx || j > g.ny) return;
   const long p = gix(g, i, j, k);
-  TDiff[p] = (Visc[p] - (Real)nu) / (Real)(double)0.6f + (Real)nu_scalar;
+  store_one_layer(g, TDiff, i, j, k, (Visc[p] - (Real)nu) / (Real)(double)0.6f + (Real)nu_scalar);
 }
 
 template <typename Real>

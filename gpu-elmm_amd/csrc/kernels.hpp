@@ -19,10 +19,12 @@ template <typename T> void launch_bound_uvw(const Geo &g, T *U, T *V, T *W, hipS
 long ghost_shell_cells(const Geo &g, int c);
 int ghost_delta_build(const Geo &g, int c, const int32_t *ijk, int n, uint8_t *mark, long long *list, int cap,
                       int *count, hipStream_t st);
-// Re-applies the ghost rules of the concatenated lists (n[0] for U, n[1] for
-// V, n[2] for W).
-template <typename T>
-void launch_ghost_delta(T *U, T *V, T *W, const long long *list, const int n[3], hipStream_t st);
+// The z ghost layers of U, V, W and P, which complete BoundUVW and Bound_Pr
+// after a projection that wrote the x and y ghost cells.
+template <typename T> void launch_bound_z(const Geo &g, T *U, T *V, T *W, T *P, hipStream_t st);
+// The interior cell whose value (negated with neg, or zero) BoundUVW gives
+// to cell (i, j, k) of component c; false when it maps to no interior cell.
+bool ghost_source(const Geo &g, int c, int i, int j, int k, int src[3], int &neg, bool &zero);
 template <typename T> void launch_bound_visc(const Geo &g, T *F, hipStream_t st);
 template <typename T> void launch_bound_scalar(const Geo &g, T *F, hipStream_t st);
 template <typename T> void launch_bound_pr(const Geo &g, T *P, hipStream_t st);
@@ -174,9 +176,12 @@ void launch_momentum_corr3(const Geo &g, const T *U, const T *V, const T *W, con
                            T *const Ustar[3], T *const U2[3], StageConst sc, const TermList tl[3],
                            const double *fluxp, const double *fluxm, hipStream_t st);
 // IBMomentum of the three components: interpolation of every point (tmp
-// holds ib[0].n + ib[1].n + ib[2].n values), then the scatter.
+// holds ib[0].n + ib[1].n + ib[2].n values), then the scatter.  ghosts (or
+// null): the ghost cells that take a point's value, nghost[c] of component c,
+// as (ghost offset, point | neg << 62) pairs, written with the scatter.
 template <typename T>
-void launch_ib_momentum(const Geo &g, const IBDev ib[3], T *U, T *V, T *W, double *tmp, hipStream_t st);
+void launch_ib_momentum(const Geo &g, const IBDev ib[3], T *U, T *V, T *W, double *tmp, const long long *ghosts,
+                        const int nghost[3], hipStream_t st);
 template <typename T>
 void launch_ib_visc_serial(const Geo &g, IBDev ib, T *Visc, const int32_t *level_ptr, int nlevels, hipStream_t st);
 template <typename T>
@@ -254,7 +259,7 @@ template <typename T>
 void launch_top_sum(const Geo &g, const T *Pr, const double *Phi, double *partial, int nblocks, hipStream_t st);
 template <typename T>
 void launch_projection(const Geo &g, T *U, T *V, T *W, T *Pr, const double *Phi, const double *partial, int nblocks,
-                       double dt2, hipStream_t st);
+                       double dt2, bool ghosts, hipStream_t st);
 template <typename T>
 void launch_max_div(const Geo &g, const T *U, const T *V, const T *W, const double *Q, double *partial, int nblocks,
                     hipStream_t st);
