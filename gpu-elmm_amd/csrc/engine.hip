@@ -1912,12 +1912,11 @@ void Engine<T>::subgrid_stresses(bool cfl) {
                  cfl ? cfl_partial.as<double>() : nullptr, cfl_blocks, stream);
     });
   sgs_prelaunched = false;
-  // ComputeViscsWM: WMPoints%ustar (the viscosity it writes is overwritten
-  // by SubgridModel)
-  if (cfg.wall_model && wmp_n)
-    timed(ELMM_T_WALL, [&] { launch_wm_ustar<T>(g, u, v, w, temp_cur(), moist_cur(), wmpdev(), cfg.nu, (T *)nullptr, stream); });
-  // constant dt with the CFL check: the step's CFL number and the divergence
-  // test, on the device (graph-safe)
+  // in one launch: the step's CFL number and divergence test (constant dt, on
+  // the device: graph-safe), ComputeUVWFluxesWM, ComputeViscsWM's
+  // WMPoints%ustar (the viscosity it writes is overwritten by SubgridModel),
+  // DivergenceWM and BoundViscosity
+  SurfaceWork<T> sw{};
   if (cfl && !cfg.variable_dt)
     sw.cfl = CflArgs{cfl_partial.as<double>(), cfl_blocks, dt_cur, cfg.cfl_max, mon};
   sw.wm = wmdev();
@@ -1995,11 +1994,6 @@ void Engine<T>::stage(int st, bool last) {
   if (nsc > 0) {
     // ScalarRK3 (src/scalars.f90:88-299) with the stage-start velocity;
     // the stage-start BoundScalar repeats the previous stage's final fill.
-    if (wmp_n)
-      timed(ELMM_T_WALL, [&] {
-        launch_wm_div(g, WMScalarPoints{wmp_n, wmp_ijk.as<int32_t>(), wmp_div.as<double>()}, prtype.as<int32_t>(), u,
-                      v, w, stream);
-      });
     for (int s = 0; s < nsc; s++) {
       timed(ELMM_T_SCALAR, [&] {
         if (zmarch_scalar)

@@ -600,14 +600,14 @@ __device__ inline void mo_dirichlet_moist(double &ustar, double &tflux, double &
 }
 
 template <typename T>
-__global__ void k_wm_fluxes(Geo g, const T *__restrict__ U_, const T *__restrict__ V_, const T *__restrict__ W_,
-                            const T *__restrict__ Temp, const T *__restrict__ Moist, WMPoints wm, double nu,
-                            int variable_z) {
+__device__ inline void wm_flux_point(const Geo &g, const T *__restrict__ U_, const T *__restrict__ V_,
+                                     const T *__restrict__ W_, const T *__restrict__ Temp,
+                                     const T *__restrict__ Moist, const WMPoints &wm, double nu, int variable_z,
+                                     int p) {
   // surface lists: evaluated in FP64 whatever the field type
   auto U = [&](long q) { return (double)U_[q]; };
   auto V = [&](long q) { return (double)V_[q]; };
   auto W = [&](long q) { return (double)W_[q]; };
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= wm.n) return;
   const int l = wm.list[p];
   const int comp = l / 6, dir = l % 6;
@@ -688,14 +688,6 @@ __global__ void k_wm_fluxes(Geo g, const T *__restrict__ U_, const T *__restrict
   wm.fluxm[p] = fluxm;
 }
 
-template <typename T>
-void launch_wm_fluxes(const Geo &g, const T *U, const T *V, const T *W, const T *Temp, const T *Moist, WMPoints wm,
-                      double nu, int variable_z, hipStream_t st) {
-  if (wm.n == 0) return;
-  hipLaunchKernelGGL(k_wm_fluxes<T>, dim3(nblk(wm.n, 256)), dim3(256), 0, st, g, U, V, W, Temp, Moist, wm, nu,
-                     variable_z);
-}
-
 // ComputeViscsWM (src/wallmodels.f90:2050-2152; neutral, wall velocity 0,
 // wallmodeltype 1): the persistent WMPoints%ustar of every scalar wall-model
 // point from the cell-centred two-point velocity (2069-2071), by
@@ -704,10 +696,10 @@ void launch_wm_fluxes(const Geo &g, const T *U, const T *V, const T *W, const T 
 // stored too; in SubgridStresses SubgridModel overwrites it, so the step
 // keeps only u*.  FP64 whatever the field type.
 template <typename T>
-__global__ void k_wm_ustar(Geo g, const T *__restrict__ U_, const T *__restrict__ V_, const T *__restrict__ W_,
-                           const T *__restrict__ Temp, const T *__restrict__ Moist, WMUstarPoints wp, double nu,
-                           T *__restrict__ Visc) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ inline void wm_ustar_point(const Geo &g, const T *__restrict__ U_, const T *__restrict__ V_,
+                                      const T *__restrict__ W_, const T *__restrict__ Temp,
+                                      const T *__restrict__ Moist, const WMUstarPoints &wp, double nu,
+                                      T *__restrict__ Visc, int p) {
   if (p >= wp.n) return;
   const int xi = wp.ijk[3 * p], yj = wp.ijk[3 * p + 1], zk = wp.ijk[3 * p + 2];
   const long q = gix(g, xi, yj, zk);
@@ -777,6 +769,14 @@ __global__ void k_wm_ustar(Geo g, const T *__restrict__ U_, const T *__restrict_
         visc = nu;
     }
   }
+  wp.ustar[p] = ustar;
+  if (Visc) Visc[q] = (T)visc;
+  // TemperatureExtra's surface source (src/scalars.f90:322-326)
+  if (wp.heat) wp.heat[p] = wp.mo.tflux[p] * wp.af[p];
+  // MoistureExtra's (src/scalars.f90:350-354)
+  if (wp.mheat) wp.mheat[p] = wp.mo.qflux[p] * wp.af[p];
+}
+
 template <typename T>
 __global__ void k_wm_ustar(Geo g, const T *__restrict__ U, const T *__restrict__ V, const T *__restrict__ W,
                            const T *__restrict__ Temp, const T *__restrict__ Moist, WMUstarPoints wp, double nu,
@@ -918,14 +918,6 @@ void launch_surface(const Geo &g, const T *U, const T *V, const T *W, const T *T
   const long ghosts = 2L * (g.nx + 2) * (g.ny + 2) + 2L * (g.nx + 2) * g.nz + 2L * g.ny * g.nz;
   hipLaunchKernelGGL(k_surface<T>, dim3(s.b_cfl + s.b_flux + s.b_ustar + s.b_div + nblk(ghosts, 256)), dim3(256), 0, st,
                      g, U, V, W, Temp, Moist, s);
-}
-
-  wp.ustar[p] = ustar;
-  if (Visc) Visc[q] = (T)visc;
-  // TemperatureExtra's surface source (src/scalars.f90:322-326)
-  if (wp.heat) wp.heat[p] = wp.mo.tflux[p] * wp.af[p];
-  // MoistureExtra's (src/scalars.f90:350-354)
-  if (wp.mheat) wp.mheat[p] = wp.mo.qflux[p] * wp.af[p];
 }
 
 template <typename T>
@@ -1158,6 +1150,12 @@ __device__ inline T momentum_rhs(const Geo &g, const T *__restrict__ U, const T 
   return diffusion<T, C>(g, Visc, F, p, w);
 }
 
+template <typename T>
+struct Mom3 {
+  T *Us[3], *U2[3];
+  const uint8_t *code[3];
+};
+
 template <typename T, int C, int VZ>
 __device__ inline void momentum_cell(const Geo &g, const T *__restrict__ U, const T *__restrict__ V,
                                      const T *__restrict__ W, const T *__restrict__ Visc, const T *__restrict__ Pr,
@@ -1178,6 +1176,9 @@ __device__ inline void momentum_cell(const Geo &g, const T *__restrict__ U, cons
   }
 }
 
+// One thread per cell, the three components in turn: their stencils share
+// the velocity, viscosity and pressure loads (one launch per component:
+// 40 + 37 + 36 us on the 256x128x128 channel in FP32).
 template <typename T, int VZ>
 __global__ void __launch_bounds__(256)
     k_momentum(Geo g, const T *__restrict__ U, const T *__restrict__ V, const T *__restrict__ W,
@@ -1298,12 +1299,6 @@ void launch_momentum_corr3(const Geo &g, const T *U, const T *V, const T *W, con
   else
     hipLaunchKernelGGL((k_momentum_corr3<T, 0>), dim3(nblk(tot, 128)), dim3(128), 0, st, g, U, V, W, Visc, Pr, a, sc,
                        fluxp, fluxm);
-template <typename T>
-struct Mom3 {
-  T *Us[3], *U2[3];
-  const uint8_t *code[3];
-};
-
 }
 
 template <typename T, int VZ>
@@ -1372,6 +1367,8 @@ __global__ void k_ib_interp(Geo g, IB3 ib, const T *__restrict__ U, const T *__r
     s = s + d.coef[t] * (double)F[gix(g, d.src[3 * t], d.src[3 * t + 1], d.src[3 * t + 2])];
   tmp[p] = s;
 }
+// The scatter, and after the points the listed ghost cells, which take the
+// same values (all that a BoundUVW would change after IBMomentum).
 template <typename T>
 __global__ void k_ib_scatter(Geo g, IB3 ib, const double *__restrict__ tmp, const long long *__restrict__ ghosts,
                              int g0, int g01, int g012, T *__restrict__ U, T *__restrict__ V, T *__restrict__ W) {
@@ -1538,6 +1535,8 @@ void launch_mass_sources(const Geo &g, TermList tl, const T *U, const T *V, cons
                               SgsWidth, int, double *, int, hipStream_t);                                          \
   template void launch_wm_fluxes<T>(const Geo &, const T *, const T *, const T *, const T *, const T *, WMPoints,  \
                                     double, int, hipStream_t);                                                     \
+  template void launch_surface<T>(const Geo &, const T *, const T *, const T *, const T *, const T *,             \
+                                  SurfaceWork<T>, hipStream_t);                                                   \
   template void launch_wm_ustar<T>(const Geo &, const T *, const T *, const T *, const T *, const T *,             \
                                    WMUstarPoints, double, T *, hipStream_t);                                       \
   template void launch_momentum<T>(const Geo &, const T *, const T *, const T *, const T *, const T *,            \

@@ -37,29 +37,6 @@ __device__ inline double nan_max(double a, double b) {
 
 }  // namespace
 
-// TimeStepLength's maximum (src/dynamics.f90:556-591) from the block maxima
-// the SGS kernel wrote at the first stage, then main.f90's divergence test
-// (src/main.f90:161-168: time_step >= 3, CFL > CFL_max; a NaN velocity makes
-// the maximum huge, src/dynamics.f90:538).
-__global__ void __launch_bounds__(256)
-    k_cfl_monitor(const double *__restrict__ partial, int nblocks, double dt, double cfl_max, StepMon *mon) {
-  double v = 0;
-  for (int b = threadIdx.x; b < nblocks; b += blockDim.x) v = nan_max(v, partial[b]);
-  const double m = block_reduce(v, nan_max);
-  if (threadIdx.x != 0) return;
-  const double cfl = m * dt;
-  const long long step = mon->step + 1;
-  mon->step = step;
-  mon->cfl_last = cfl;
-  mon->umax_last = m;
-  if (cfl_max > 0 && step >= 3 && !(cfl <= cfl_max) && mon->first_bad < 0) mon->first_bad = step;
-}
-
-void launch_cfl_monitor(const double *partial, int nblocks, double dt, double cfl_max, StepMon *mon,
-                        hipStream_t st) {
-  hipLaunchKernelGGL(k_cfl_monitor, dim3(1), dim3(256), 0, st, partial, nblocks, dt, cfl_max, mon);
-}
-
 // TMarchRK3's delta (src/tsteps.f90:188-207): per stage the mean over each
 // component's interior of |U - U2| (U the stage-start velocity, U2 the
 // projected one), summed over the components and stages, divided by dt at

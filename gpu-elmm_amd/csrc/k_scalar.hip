@@ -474,8 +474,6 @@ void launch_moist_fill(const Geo &g, const uint8_t *code, Real *q, double ref, h
   template void launch_scalar_corr<R>(const Geo &, const R *, const R *, const R *, const R *, const R *, R *, R *, \
                                       const uint8_t *, const uint8_t *, const uint8_t *, const uint8_t *,          \
                                       StageConst, TermList, const double *, const double *, hipStream_t);          \
-  template void launch_wm_div<R>(const Geo &, WMScalarPoints, const int32_t *, const R *, const R *, const R *,    \
-                                 hipStream_t);                                                                    \
   template void launch_tdiff_init<R>(const Geo &, const R *, R *, double, double, hipStream_t);                 \
   template void launch_temp_solid_fix<R>(const Geo &, const int32_t *, int, const int32_t *, R *, hipStream_t);  \
   template void launch_moist_fill<R>(const Geo &, const uint8_t *, R *, double, hipStream_t);                      \

@@ -191,9 +191,6 @@ void launch_mass_sources(const Geo &g, TermList tl, const T *U, const T *V, cons
 
 // scalar (k_scalar.hip); R = field type (double or float)
 template <typename R>
-void launch_wm_div(const Geo &g, WMScalarPoints p, const int32_t *prtype, const R *U, const R *V, const R *W,
-                   hipStream_t st);
-template <typename R>
 void launch_scalar(const Geo &g, const R *U, const R *V, const R *W, const R *TDiff, const R *S, R *Snew, R *Sadv,
                    const uint8_t *code, const uint8_t *mx, const uint8_t *my, const uint8_t *mz, StageConst sc,
                    hipStream_t st);
@@ -273,8 +270,31 @@ struct StepMon {
   long long step;         // steps counted by the CFL monitor
   long long first_bad;    // first step (1-based) with CFL > CFL_max, -1 none
 };
-void launch_cfl_monitor(const double *partial, int nblocks, double dt, double cfl_max, StepMon *mon,
-                        hipStream_t st);
+// The CFL monitor's inputs (mon null: off).
+struct CflArgs {
+  const double *partial;  // the SGS kernel's block maxima
+  int nblocks;
+  double dt, cfl_max;
+  StepMon *mon;
+};
+// Stage-start work on lists and surfaces in one launch (k_momentum.hip): the
+// CFL monitor, the wall fluxes, u* and the velocity divergence of the scalar
+// wall-model points (each off with no points) and the viscosity's ghost
+// layer.  b_*: blocks of each part, set by the launcher.
+template <typename T>
+struct SurfaceWork {
+  CflArgs cfl;
+  WMPoints wm;
+  WMUstarPoints wp;
+  WMScalarPoints div;
+  const int32_t *prtype;
+  T *visc;
+  double nu;
+  int b_cfl, b_flux, b_ustar, b_div;
+};
+template <typename T>
+void launch_surface(const Geo &g, const T *U, const T *V, const T *W, const T *Temp, const T *Moist,
+                    SurfaceWork<T> s, hipStream_t st);
 int delta_blocks(const Geo &g);
 template <typename T>
 void launch_delta(const Geo &g, const T *U, const T *U2, const T *V, const T *V2, const T *W, const T *W2,
