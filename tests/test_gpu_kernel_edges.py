@@ -1,0 +1,115 @@
+"""Grids at the edges of the kernels' tiles, tables and walks against the
+oracle, bit for bit in the FP64 form: the FP64 form restates the reference's
+operations in its order (src/poisson.f90:76-140, src/cds.f90:46-153), so the
+tolerance is zero wherever the oracle's own order is the definition."""
+import numpy as np
+import pytest
+
+from elmm_amd import capi, cases
+from helpers import compare_state
+from oracle_py import Oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(cfg, steps=2, cuboids=(), sources=(), seed=7):
+    case = capi.Case(cfg, cuboids=cuboids, sources=sources)
+    f = cases.initial_fields(cfg, u0=1.5, amp=0.2, seed=seed)
+    o, s = Oracle(cfg, case), capi.Solver(cfg, case)
+    for x in (o, s):
+        cases.upload_initial(x, cfg, f)
+        x.init()
+        x.step(steps)
+    return o, s
+
+
+def _same(o, s, cfg):
+    err = compare_state(s, o, cfg)
+    print(f"{cfg.nx}x{cfg.ny}x{cfg.nz}: {err}", flush=True)
+    assert max(err.values()) == 0.0, err
+
+
+# every grouping of the radix-3 and radix-2 stages (one group up to 9, then
+# 9 9 3, 9 9 6, 6 4 4, 9 8 .. 972 = 9 9 3 4), one to 64 lines per block, and
+# row counts that leave the last block partly empty
+@pytest.mark.parametrize("nx,ny,nz", [(6, 9, 5), (12, 27, 4), (18, 24, 7), (81, 54, 5), (162, 36, 4), (486, 6, 4),
+                                      (8, 243, 5), (768, 12, 4), (972, 4, 4), (4, 972, 4), (64, 576, 4)])
+def test_mixed_radix_groups(require_gpu, nx, ny, nz):
+    cfg = cases.uniform_config(nx, ny, nz, dx=1.0, dt=0.02)
+    _same(*_run(cfg, steps=1), cfg)
+
+
+# the z solve's pivot table at the shortest columns, a partly filled group of
+# modes, column lengths about its load groups of 8, the longest that its LDS
+# takes and, beyond, the kernel that divides
+@pytest.mark.parametrize("nx,ny,nz", [(8, 6, 4), (6, 9, 5), (16, 4, 7), (8, 12, 8), (16, 9, 9), (4, 4, 33),
+                                      (8, 6, 350), (4, 8, 600)])
+def test_z_solve_lengths(require_gpu, nx, ny, nz):
+    cfg = cases.uniform_config(nx, ny, nz, dx=1.0, dt=0.02)
+    _same(*_run(cfg), cfg)
+
+
+# the line sweep stages columns in groups of 8 layers and 16 modes; stretched z
+@pytest.mark.parametrize("nx,ny,nz", [(12, 20, 9), (36, 8, 22), (16, 16, 15)])
+def test_multigrid_column_lengths(require_gpu, nx, ny, nz):
+    cfg = cases.channel_config(nx, ny, nz, poisson_solver=capi.POISSON_MG)
+    case = capi.Case(cfg)
+    f = cases.channel_fields(cfg, seed=4)
+    o, s = Oracle(cfg, case), capi.Solver(cfg, case)
+    for x in (o, s):
+        cases.upload_initial(x, cfg, f)
+        x.init()
+        x.step(1)
+    _same(o, s, cfg)
+
+
+# walk lengths and tiles of the z-marching kernels: layers that no walk
+# divides, rows and columns that leave tiles partly empty, two scalars
+@pytest.mark.parametrize("nx,ny,nz", [(64, 8, 5), (66, 10, 17), (128, 12, 31), (36, 64, 65)])
+def test_walk_remainders(require_gpu, nx, ny, nz):
+    kw = {} if nx % 11 else dict(poisson_solver=capi.POISSON_MG)
+    cfg = cases.uniform_config(nx, ny, nz, dx=1.0, dt=0.02, nscalars=2, **kw)
+    _same(*_run(cfg, sources=[(2.5, 2.5, 0.5, 1.0, 0), (nx - 1.5, 3.5, 1.5, 2.0, 1)]), cfg)
+
+
+def _periodic_images(a, nx, ny):
+    i = 3 + (np.arange(nx + 6) - 3) % nx
+    j = 3 + (np.arange(ny + 6) - 3) % ny
+    return a[i][:, j]
+
+
+# obstacles across the periodic edges: the kernels that write a value there
+# (projection, immersed-boundary points, points inside solids) write its
+# images too; 4 and 5 cells: a cell has images on both sides
+@pytest.mark.parametrize("nx,ny,nz", [(4, 8, 6), (8, 4, 6), (24, 18, 8), (64, 32, 12)])
+def test_ghosts_are_images(require_gpu, nx, ny, nz):
+    cfg = cases.uniform_config(nx, ny, nz, dx=1.0, dt=0.02, nscalars=1)
+    cub = [(-1.2, 1.2, -1.2, 1.2, 0.0, 2.2), (nx - 1.4, nx + 1.4, ny / 2 - 1.1, ny / 2 + 1.1, 0.0, 3.1)]
+    o, s = _run(cfg, cuboids=cub)
+    _same(o, s, cfg)
+    for c in range(3):
+        a = s.download(c)
+        np.testing.assert_array_equal(a[:, :, 3:3 + nz], _periodic_images(a, nx, ny)[:, :, 3:3 + nz])
+        np.testing.assert_array_equal(a, o.download(c))
+
+
+# boxes of a field: inside it, exactly it, beyond it; fields of less than a
+# slot, of one row per slab and of several slots per thread
+@pytest.mark.parametrize("n", [(6, 4, 4), (48, 24, 20), (192, 144, 96)])
+@pytest.mark.parametrize("prec", [capi.FP64, capi.FP32_REFINED])
+def test_field_boxes(require_gpu, n, prec):
+    cfg = capi.with_precision(cases.uniform_config(*n, dx=1.0, dt=0.02), prec)
+    s = capi.Solver(cfg, capi.Case(cfg))
+    rng = np.random.default_rng(3)
+    full = rng.standard_normal(capi.ghosted_shape(cfg)).astype(np.float32).astype(np.float64)
+    s.upload(0, full)
+    np.testing.assert_array_equal(s.download(0), full)
+    part = rng.standard_normal((n[0] - 1, n[1], n[2] + 1)).astype(np.float32).astype(np.float64)
+    s.upload(0, part, lb=1)
+    full[3:2 + n[0], 3:3 + n[1], 3:4 + n[2]] = part
+    np.testing.assert_array_equal(s.download(0), full)
+    np.testing.assert_array_equal(s.download(0, lb=2, shape=(2, 3, 3)), full[4:6, 4:7, 4:7])
+    wide = s.download(0, lb=-4, shape=tuple(x + 10 for x in n))
+    np.testing.assert_array_equal(wide[2:-2, 2:-2, 2:-2], full)
+    wide[2:-2, 2:-2, 2:-2] = 0
+    assert not wide.any()
