@@ -262,33 +262,65 @@ __global__ void __launch_bounds__(256) k_mg_prolong(MgLevel Cs, MgLevel F) {
 // Fourier sums in x, then y (twiddles w(q) = (cos 2 pi q/N, -sin 2 pi q/N)),
 // a tridiagonal elimination in z per mode (the (0, 0) mode integrated as the
 // singular Neumann problem with x_1 = 0), conjugate sums over y, then x.
-// Work arrays Y, X (complex, nx ny nz) and cp (nx ny nz) in global memory.
-__global__ void __launch_bounds__(256) k_mg_coarse(MgLevel L, MgCoarse C, const double *__restrict__ az,
-                                                   const double *__restrict__ cz, const double *__restrict__ dzPr,
-                                                   const double *__restrict__ dzW) {
+// The right-hand side, the work arrays Y, X (complex, nx ny nz) and cp (nx ny
+// nz, which takes the right-hand side's place) and the tables are held in LDS
+// where they fit (SH), else in global memory: the sums and the elimination
+// are chains of dependent reads, 8x4x64 100 us from global memory by 256
+// threads, 34 us from LDS by 1024.
+constexpr int kMgCoarseThreads = 1024;
+constexpr size_t mg_coarse_lds(long n, int nx, int ny, int nz) {
+  return (size_t)(n * 5 + 2 * (nx + ny) + 2 * nz) * sizeof(double);
+}
+template <bool SH>
+__global__ void __launch_bounds__(SH ? kMgCoarseThreads : 256)
+    k_mg_coarse(MgLevel L, MgCoarse C, const double *__restrict__ gaz, const double *__restrict__ gcz,
+                const double *__restrict__ dzPr, const double *__restrict__ dzW) {
+  extern __shared__ __align__(16) double sm[];
   const int nx = L.nx, ny = L.ny, nz = L.nz;
-  const long plane = (long)nx * ny, n = plane * nz;
-  double2 *Y = C.Y, *X = C.X;
-  for (long q = threadIdx.x; q < n; q += blockDim.x) {
-    const int m = (int)(q % nx), j = (int)((q / nx) % ny), k = (int)(q / plane);
+  const int plane = nx * ny, n = plane * nz;
+  double2 *Y = SH ? reinterpret_cast<double2 *>(sm) : C.Y, *X = SH ? Y + n : C.X;
+  double *cp = SH ? sm + 4 * (long)n : C.cp;
+  double *tab = sm + 5 * (long)n;
+  const double *rhs = SH ? cp : L.rhs;
+  const double *cx = SH ? tab : C.cx, *sx = SH ? cx + nx : C.sx;
+  const double *cy = SH ? sx + nx : C.cy, *sy = SH ? cy + ny : C.sy;
+  const double *az = SH ? sy + ny : gaz, *cz = SH ? az + nz : gcz;
+  if (SH) {
+    for (int q = threadIdx.x; q < n; q += blockDim.x) cp[q] = L.rhs[q];
+    for (int q = threadIdx.x; q < nx; q += blockDim.x) {
+      tab[q] = C.cx[q];
+      tab[nx + q] = C.sx[q];
+    }
+    for (int q = threadIdx.x; q < ny; q += blockDim.x) {
+      tab[2 * nx + q] = C.cy[q];
+      tab[2 * nx + ny + q] = C.sy[q];
+    }
+    for (int q = threadIdx.x; q < nz; q += blockDim.x) {
+      tab[2 * (nx + ny) + q] = gaz[q];
+      tab[2 * (nx + ny) + nz + q] = gcz[q];
+    }
+    __syncthreads();
+  }
+  // tq = (m i) mod nx by steps
+  const auto next = [](int tq, int m, int len) { return tq + m >= len ? tq + m - len : tq + m; };
+  for (int q = threadIdx.x; q < n; q += blockDim.x) {
+    const int row = q / nx, m = q - row * nx;
     double ar = 0, ai = 0;
-    for (int i = 0; i < nx; i++) {
-      const int tq = (m * i) % nx;
-      const double r = L.rhs[i + (long)j * nx + (long)k * plane];
-      const double pr = r * C.cx[tq] - 0.0 * C.sx[tq], pi = r * C.sx[tq] + 0.0 * C.cx[tq];
+    for (int i = 0, tq = 0; i < nx; i++, tq = next(tq, m, nx)) {
+      const double r = rhs[i + row * nx];
+      const double pr = r * cx[tq] - 0.0 * sx[tq], pi = r * sx[tq] + 0.0 * cx[tq];
       ar = ar + pr;
       ai = ai + pi;
     }
     Y[q] = make_double2(ar, ai);
   }
   __syncthreads();
-  for (long q = threadIdx.x; q < n; q += blockDim.x) {
-    const int m = (int)(q % nx), nn = (int)((q / nx) % ny), k = (int)(q / plane);
+  for (int q = threadIdx.x; q < n; q += blockDim.x) {
+    const int row = q / nx, m = q - row * nx, k = row / ny, nn = row - k * ny;
     double ar = 0, ai = 0;
-    for (int j = 0; j < ny; j++) {
-      const int tq = (nn * j) % ny;
-      const double2 y = Y[m + (long)j * nx + (long)k * plane];
-      const double pr = y.x * C.cy[tq] - y.y * C.sy[tq], pi = y.x * C.sy[tq] + y.y * C.cy[tq];
+    for (int j = 0, tq = 0; j < ny; j++, tq = next(tq, nn, ny)) {
+      const double2 y = Y[m + j * nx + k * plane];
+      const double pr = y.x * cy[tq] - y.y * sy[tq], pi = y.x * sy[tq] + y.y * cy[tq];
       ar = ar + pr;
       ai = ai + pi;
     }
@@ -301,8 +333,8 @@ __global__ void __launch_bounds__(256) k_mg_coarse(MgLevel L, MgCoarse C, const 
     if (m == 0 && nn == 0) {
       double Gr = 0, Gi = 0, xr = 0, xi = 0;
       for (int k = 1; k <= nz; k++) {
-        const double2 d = col[(long)(k - 1) * plane];
-        col[(long)(k - 1) * plane] = make_double2(xr, xi);
+        const double2 d = col[(k - 1) * plane];
+        col[(k - 1) * plane] = make_double2(xr, xi);
         if (k < nz) {
           Gr = Gr + d.x * dzPr[k];
           Gi = Gi + d.y * dzPr[k];
@@ -314,34 +346,41 @@ __global__ void __launch_bounds__(256) k_mg_coarse(MgLevel L, MgCoarse C, const 
     }
     const double lam = C.lam[mode];  // host table (the host's sin)
     double cprev = 0, dr = 0, di = 0;
+    double2 d = col[0];
+    double a = az[0], c = cz[0];
     for (int k = 0; k < nz; k++) {
-      const double b = (lam - az[k]) - cz[k];
-      const double den = b - az[k] * cprev;
-      const double cpk = cz[k] / den;
-      C.cp[mode + (long)k * plane] = cpk;
-      const double2 d = col[(long)k * plane];
-      dr = (d.x - az[k] * dr) / den;
-      di = (d.y - az[k] * di) / den;
-      col[(long)k * plane] = make_double2(dr, di);
+      // the next level's inputs before this level's chain
+      const int kn = min(k + 1, nz - 1);
+      const double2 dn = col[kn * plane];
+      const double an = az[kn], cn = cz[kn];
+      const double b = (lam - a) - c;
+      const double den = b - a * cprev;
+      const double cpk = c / den;
+      dr = (d.x - a * dr) / den;
+      di = (d.y - a * di) / den;
+      cp[mode + k * plane] = cpk;
+      col[k * plane] = make_double2(dr, di);
       cprev = cpk;
+      d = dn;
+      a = an;
+      c = cn;
     }
     double xr = dr, xi = di;
     for (int k = nz - 2; k >= 0; k--) {
-      const double2 dp = col[(long)k * plane];
-      const double cpk = C.cp[mode + (long)k * plane];
+      const double2 dp = col[k * plane];
+      const double cpk = cp[mode + k * plane];
       xr = dp.x - cpk * xr;
       xi = dp.y - cpk * xi;
-      col[(long)k * plane] = make_double2(xr, xi);
+      col[k * plane] = make_double2(xr, xi);
     }
   }
   __syncthreads();
-  for (long q = threadIdx.x; q < n; q += blockDim.x) {
-    const int m = (int)(q % nx), j = (int)((q / nx) % ny), k = (int)(q / plane);
+  for (int q = threadIdx.x; q < n; q += blockDim.x) {
+    const int row = q / nx, m = q - row * nx, k = row / ny, j = row - k * ny;
     double ar = 0, ai = 0;
-    for (int nn = 0; nn < ny; nn++) {
-      const int tq = (nn * j) % ny;
-      const double2 x = X[m + (long)nn * nx + (long)k * plane];
-      const double wr = C.cy[tq], wi = -C.sy[tq];
+    for (int nn = 0, tq = 0; nn < ny; nn++, tq = next(tq, j, ny)) {
+      const double2 x = X[m + nn * nx + k * plane];
+      const double wr = cy[tq], wi = -sy[tq];
       const double pr = x.x * wr - x.y * wi, pi = x.x * wi + x.y * wr;
       ar = ar + pr;
       ai = ai + pi;
@@ -350,13 +389,12 @@ __global__ void __launch_bounds__(256) k_mg_coarse(MgLevel L, MgCoarse C, const 
   }
   __syncthreads();
   const double scale = 1.0 / (double)plane;
-  for (long q = threadIdx.x; q < n; q += blockDim.x) {
-    const int i = (int)(q % nx), j = (int)((q / nx) % ny), k = (int)(q / plane);
+  for (int q = threadIdx.x; q < n; q += blockDim.x) {
+    const int row = q / nx, i = q - row * nx;
     double acc = 0;
-    for (int m = 0; m < nx; m++) {
-      const int tq = (m * i) % nx;
-      const double2 y = Y[m + (long)j * nx + (long)k * plane];
-      const double wr = C.cx[tq], wi = -C.sx[tq];
+    for (int m = 0, tq = 0; m < nx; m++, tq = next(tq, i, nx)) {
+      const double2 y = Y[m + row * nx];
+      const double wr = cx[tq], wi = -sx[tq];
       acc = acc + (y.x * wr - y.y * wi);
     }
     L.phi[q] = acc * scale;
@@ -405,7 +443,13 @@ void launch_mg_prolong(const MgLevel &Cs, const MgLevel &F, hipStream_t st) {
 
 void launch_mg_coarse(const MgLevel &L, const MgCoarse &C, const double *az, const double *cz, const double *dzPr,
                       const double *dzW, hipStream_t st) {
-  hipLaunchKernelGGL(k_mg_coarse, dim3(1), dim3(256), 0, st, L, C, az, cz, dzPr, dzW);
+  const size_t sh = mg_coarse_lds((long)L.nx * L.ny * L.nz, L.nx, L.ny, L.nz);
+  if (sh <= 160 * 1024) {
+    if (sh > 65536) (void)lds_limit_raise((const void *)k_mg_coarse<true>, sh);
+    hipLaunchKernelGGL(k_mg_coarse<true>, dim3(1), dim3(kMgCoarseThreads), sh, st, L, C, az, cz, dzPr, dzW);
+  } else {
+    hipLaunchKernelGGL(k_mg_coarse<false>, dim3(1), dim3(256), 0, st, L, C, az, cz, dzPr, dzW);
+  }
 }
 
 template void launch_mg_rhs<double>(const Geo &, const double *, const double *, const double *, const double *,
