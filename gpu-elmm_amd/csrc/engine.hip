@@ -985,6 +985,11 @@ void Engine<T>::setup_mg() {
     mg_bufs.emplace_back(new DevBuf);
     mg_bufs.back()->alloc(n * sizeof(double));
     v.rhs = mg_bufs.back()->as<double>();
+    if (l < L - 1 && mg_smooth_wanted(v)) {
+      mg_bufs.emplace_back(new DevBuf);
+      mg_bufs.back()->alloc(n * sizeof(double));
+      v.phi2 = mg_bufs.back()->as<double>();
+    }
     double *den = &tab[(size_t)(2 * l) * nz], *e = &tab[(size_t)(2 * l + 1) * nz];
     double eprev = 0;
     for (int k = 1; k <= nz; k++) {
@@ -1061,17 +1066,22 @@ void Engine<T>::mg_vcycle(int l) {
     return;
   }
   const double *den = mg_tab.as<double>() + (size_t)(2 * l) * nz, *e = den + nz;
-  auto smooth = [&] {
+  auto smooth = [&](const MgLevel *coarse) {
+    if (mg[l].phi2) {
+      launch_mg_smooth(mg[l], coarse, az, den, e, stream);
+      std::swap(mg[l].phi, mg[l].phi2);
+      return;
+    }
+    if (coarse) launch_mg_prolong(*coarse, mg[l], stream);
     for (int s = 0; s < 2; s++) {
       launch_mg_sweep(mg[l], az, den, e, 0, stream);
       launch_mg_sweep(mg[l], az, den, e, 1, stream);
     }
   };
-  smooth();
+  smooth(nullptr);
   launch_mg_restrict(mg[l], mg[l + 1], az, cz, stream);
   mg_vcycle(l + 1);
-  launch_mg_prolong(mg[l + 1], mg[l], stream);
-  smooth();
+  smooth(&mg[l + 1]);
 }
 
 // PoissMG's loop (src/multigrid.f90:1161-1168): from P = 0, V-cycles until

@@ -22,6 +22,7 @@
 //   coarsest level: exact, by discrete Fourier sums in x and y and a
 //     tridiagonal elimination in z per mode (k_mg_coarse).
 #include <cmath>
+#include <type_traits>
 
 #include "device_common.hpp"
 #include "kernels.hpp"
@@ -96,18 +97,121 @@ __global__ void __launch_bounds__(256) k_mg_zero(double *__restrict__ a, long n)
 // COLS columns and all levels with every load in flight, keeps the columns in
 // LDS for the two passes, and writes them back.  (One thread per column
 // loading as it went: 30 us a sweep of 128x64 columns of 64 levels, bound by
-// a memory round trip per four levels; staged about 10.)
-// Levels are padded to whole groups of ZB (padding: zeros, whose sweeps stay
-// zero), so the chain carries no conditions and a group's operands are
+// a memory round trip per four levels; staged about 9.)
+// Levels are padded to whole groups of ZB, so the chain carries no conditions and a group's operands are
 // fetched while the previous group is worked through.
-constexpr int kMgCols = 16, kMgThreads = 256, ZB = 8;
+constexpr int kMgCols = 16, kMgThreads = 256, ZB = 4;
 __host__ __device__ constexpr int mg_pad(int nz) { return (nz + ZB - 1) / ZB * ZB; }
+// Tables of a sweep in LDS: az, den, RN(1/den) and e of each level.
+struct MgTab {
+  double *az, *den, *rden, *e;
+};
+__device__ inline MgTab mg_tab_at(double *p, int np) { return MgTab{p, p + np, p + 2 * np, p + 3 * np}; }
+template <int TH>
+__device__ inline void mg_tab_fill(MgTab t, const double *__restrict__ az, const double *__restrict__ den,
+                                   const double *__restrict__ e, int nz, int np) {
+  for (int k = threadIdx.x; k < np; k += TH) {
+    const int kc = min(k, nz - 1);
+    const double a = az[kc], d = den[kc], ek = e[kc];
+    t.az[k] = k < nz ? a : 0.0;
+    t.den[k] = k < nz ? d : 1.0;
+    t.rden[k] = k < nz ? (fabs(d) >= 0x1p-200 && fabs(d) <= 0x1p200 ? 1.0 / d : 0.0) : 1.0;
+    t.e[k] = k < nz ? ek : 0.0;
+  }
+}
+
+// Thomas elimination up a column of np levels at x[k * S] (h - rhs on entry,
+// 1 above level nz; P on return) and back down.
+// A column is one lane of one wave, whose time is its instructions one after
+// another.  The quotient is formed from r = RN(1/d) in 5 instead of 11: q0 =
+// RN(x r) is within two ulp of x/d, one Newton step gives a q1 within one
+// ulp, and then RN(q1 + (x - q1 d) r) is the correctly rounded quotient (P.
+// Markstein, IBM J. Res. Dev. 34, 1990), as long as no remainder underflows:
+// a group of levels with a quotient outside 2^-700..2^700 (zeros too: their
+// sign; r = 0 marks a d outside 2^-200..2^200) is done again with divisions.
+template <int S>
+__device__ inline void mg_column(double *x, MgTab tb, int nz, int np) {
+  double xc[ZB], ac[ZB], dc[ZB], rc[ZB];
+  double gv = 0;
+  // 2^-700 <= |v| < 2^700 as one unsigned range of the upper word
+  constexpr unsigned lo = (1023u - 700) << 20, range = 1400u << 20;
+  auto fetch = [&](int k0, const double *p, double *xo, double *ao) {
+#pragma unroll
+    for (int b = 0; b < ZB; b++) {
+      xo[b] = x[(k0 + b) * S];
+      ao[b] = p[k0 + b];
+    }
+  };
+  auto fetch_d = [&](int k0, double *dd, double *rr) {
+#pragma unroll
+    for (int b = 0; b < ZB; b++) {
+      dd[b] = tb.den[k0 + b];
+      rr[b] = tb.rden[k0 + b];
+    }
+  };
+  fetch(0, tb.az, xc, ac);
+  fetch_d(0, dc, rc);
+#pragma unroll 2
+  for (int k0 = 0; k0 < np; k0 += ZB) {
+    double xn[ZB], an[ZB], dn[ZB], rn[ZB], g[ZB];
+    const int kn = min(k0 + ZB, np - ZB);
+    fetch(kn, tb.az, xn, an);
+    fetch_d(kn, dn, rn);
+    const double g0 = gv;
+    unsigned far = 0;
+#pragma unroll
+    for (int b = 0; b < ZB; b++) {
+      const double t = xc[b] + ac[b] * gv;
+      const double q0 = t * rc[b], q1 = fma(fma(-q0, dc[b], t), rc[b], q0);
+      gv = fma(fma(-q1, dc[b], t), rc[b], q1);
+      far = max(far, ((unsigned)__double2hiint(gv) & 0x7fffffffu) - lo);
+      g[b] = gv;
+    }
+    if (far >= range) {
+      gv = g0;
+#pragma unroll
+      for (int b = 0; b < ZB; b++) {
+        gv = (xc[b] + ac[b] * gv) / dc[b];
+        g[b] = gv;
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < ZB; b++) {
+      x[(k0 + b) * S] = g[b];
+      xc[b] = xn[b];
+      ac[b] = an[b];
+      dc[b] = dn[b];
+      rc[b] = rn[b];
+    }
+  }
+  // P of the top level is its g: e is 0 there, and v = -0 above it leaves
+  // any sum unchanged
+  for (int k = nz; k < np; k++) x[k * S] = -0.0;
+  double v = -0.0;
+  fetch(np - ZB, tb.e, xc, ac);
+#pragma unroll 2
+  for (int k0 = np - ZB; k0 >= 0; k0 -= ZB) {
+    double xn[ZB], an[ZB];
+    fetch(max(k0 - ZB, 0), tb.e, xn, an);
+#pragma unroll
+    for (int b = ZB - 1; b >= 0; b--) {
+      v = xc[b] + ac[b] * v;
+      x[(k0 + b) * S] = v;
+    }
+#pragma unroll
+    for (int b = 0; b < ZB; b++) {
+      xc[b] = xn[b];
+      ac[b] = an[b];
+    }
+  }
+}
+
 __global__ void __launch_bounds__(kMgThreads) k_mg_sweep(MgLevel L, const double *__restrict__ az,
                                                          const double *__restrict__ den,
                                                          const double *__restrict__ e, int color) {
-  extern __shared__ double hs[];  // [np][kMgCols], then az, den and e [np]
+  extern __shared__ double hs[];  // [np][kMgCols], then the tables
   const int half = L.nx / 2, ncol = half * L.ny, nx = L.nx, nz = L.nz, np = mg_pad(nz);
-  double *saz = hs + np * kMgCols, *sden = saz + np, *se = sden + np;
+  const MgTab tb = mg_tab_at(hs + np * kMgCols, np);
   const int l = threadIdx.x % kMgCols, t = blockIdx.x * kMgCols + l;
   const int tc = min(t, ncol - 1);
   const int j = tc / half + 1, ii = tc - (j - 1) * half;
@@ -137,74 +241,123 @@ __global__ void __launch_bounds__(kMgThreads) k_mg_sweep(MgLevel L, const double
       for (int u = 0; u < NK; u++) {
         const int k = k0 + u * SK;
         const double h = L.ax * (w[u] + ea[u]) + L.ay * (so[u] + no[u]);
-        if (k < np) hs[k * kMgCols + l] = k < nz ? h - r[u] : -0.0;
+        if (k < np) hs[k * kMgCols + l] = k < nz ? h - r[u] : 1.0;
       }
     }
-    for (int k = threadIdx.x; k < np; k += kMgThreads) {
-      const int kc = min(k, nz - 1);
-      const double a = az[kc], d = den[kc], ek = e[kc];
-      saz[k] = k < nz ? a : 0.0;
-      sden[k] = k < nz ? d : 1.0;
-      se[k] = k < nz ? ek : 0.0;
-    }
+    mg_tab_fill<kMgThreads>(tb, az, den, e, nz, np);
   }
   __syncthreads();
-  if (threadIdx.x < kMgCols) {
-    double *x = hs + l;
-    double xc[ZB], ac[ZB], dc[ZB];
-    double gv = 0;
-    auto fetch = [&](int k0, const double *p, double *xo, double *ao) {
-#pragma unroll
-      for (int b = 0; b < ZB; b++) {
-        xo[b] = x[(k0 + b) * kMgCols];
-        ao[b] = p[k0 + b];
-      }
-    };
-    fetch(0, saz, xc, ac);
-#pragma unroll
-    for (int b = 0; b < ZB; b++) dc[b] = sden[b];
-    for (int k0 = 0; k0 < np; k0 += ZB) {
-      double xn[ZB], an[ZB], dn[ZB];
-      const int kn = min(k0 + ZB, np - ZB);
-      fetch(kn, saz, xn, an);
-#pragma unroll
-      for (int b = 0; b < ZB; b++) dn[b] = sden[kn + b];
-#pragma unroll
-      for (int b = 0; b < ZB; b++) {
-        gv = (xc[b] + ac[b] * gv) / dc[b];
-        x[(k0 + b) * kMgCols] = gv;
-      }
-#pragma unroll
-      for (int b = 0; b < ZB; b++) {
-        xc[b] = xn[b];
-        ac[b] = an[b];
-        dc[b] = dn[b];
-      }
-    }
-    // P of the top level is its g: e is 0 there, and v = -0 above it leaves
-    // any sum unchanged
-    for (int k = nz; k < np; k++) x[k * kMgCols] = -0.0;
-    double v = -0.0;
-    fetch(np - ZB, se, xc, ac);
-    for (int k0 = np - ZB; k0 >= 0; k0 -= ZB) {
-      double xn[ZB], an[ZB];
-      fetch(max(k0 - ZB, 0), se, xn, an);
-#pragma unroll
-      for (int b = ZB - 1; b >= 0; b--) {
-        v = xc[b] + ac[b] * v;
-        x[(k0 + b) * kMgCols] = v;
-      }
-#pragma unroll
-      for (int b = 0; b < ZB; b++) {
-        xc[b] = xn[b];
-        ac[b] = an[b];
-      }
-    }
-  }
+  if (threadIdx.x < kMgCols) mg_column<kMgCols>(hs + l, tb, nz, np);
   __syncthreads();
   if (t < ncol) {
 #pragma unroll 4
     for (int k = threadIdx.x / kMgCols; k < nz; k += kMgThreads / kMgCols) P[c + (long)k * plane] = hs[k * kMgCols + l];
+  }
+}
+
+// Both colours' sweeps twice over, a whole smoothing, in one launch: a block
+// owns a tile of kMgTile x kMgTile columns, holds it with a ring of 4 columns
+// in LDS and sweeps everything within 3 columns of the tile.  What a sweep
+// leaves right shrinks by one ring per colour: after the first it reaches 3
+// columns out, after the fourth it is the tile, which the block writes to the
+// level's other array (its neighbours still read this one).  Columns of
+// colour 0 are written before they are read, so only colour 1 is loaded; with
+// PRO the coarse correction is added in that load (see k_mg_prolong).
+// The columns of a colour are solved in place: a column's own values are not
+// read by its sweep.  (Columns of the outer rings take unset or outdated
+// neighbours in; what comes of that stays out of the tile.)
+// 128x64 / 64x32 / 16x8 columns of 64 levels: four sweeps and the prolongation
+// 45 us in five launches, 50 / 33 / 31 here, of which 10 are loads and stores,
+// 5 the sums and 16 the four columns' chains.
+constexpr int kMgTile = 4, kMgReg = kMgTile + 8, kMgRegCols = kMgReg * kMgReg;
+constexpr int kMgHalf = (kMgTile + 6) * (kMgTile + 6) / 2;  // swept columns of a colour
+constexpr int kMgSmoothThreads = 512;
+constexpr size_t mg_smooth_lds(int nz) { return (size_t)mg_pad(nz) * (kMgRegCols + 4) * sizeof(double); }
+// Where: two blocks in a CU's LDS (nz <= 68) and at most two per CU (512).
+// ms a step of the channel, smoothings whole on levels up to 0 / 128 / 512 /
+// 2048 tiles: 128x128x32 16.2 / 14.6 / 13.7 / 14.2, 128x64x64 12.2 / 11.7 /
+// 11.8 / 11.8, 256x128x64 18.3 / 17.6 / 17.8 / 23.5; with one block per CU
+// 128x64x128 19.8 / 19.8 / 22.5 / 22.5.
+constexpr long kMgSmoothMaxTiles = 512;
+constexpr int kMgMaxNr = 7;
+static_assert(2 * mg_smooth_lds(68) <= 160 * 1024 && 2 * mg_smooth_lds(69) > 160 * 1024 &&
+                  kMgHalf * 68 <= kMgMaxNr * kMgSmoothThreads,
+              "values of a colour per thread at the largest nz");
+// NR: right-hand-side values of a colour per thread
+template <int NR, bool PRO>
+__global__ void __launch_bounds__(kMgSmoothThreads, 4)
+    k_mg_smooth(MgLevel L, MgLevel Cs, const double *__restrict__ az, const double *__restrict__ den,
+                const double *__restrict__ e) {
+  extern __shared__ double hs[];  // [np][kMgRegCols], then the tables
+  constexpr int S = kMgRegCols, TH = kMgSmoothThreads;
+  const int nx = L.nx, ny = L.ny, nz = L.nz, np = mg_pad(nz), tid = threadIdx.x;
+  const MgTab tb = mg_tab_at(hs + np * S, np);
+  const int tx = blockIdx.x % (nx / kMgTile), ty = blockIdx.x / (nx / kMgTile);
+  const int i0 = tx * kMgTile - 4, j0 = ty * kMgTile - 4;  // level column of the region's column (0, 0)
+  const long plane = (long)nx * ny;
+  // nx, ny are multiples of 4 and at least 8: one wrap suffices
+  const auto wrapi = [&](int i) { return i < 0 ? i + nx : i >= nx ? i - nx : i; };
+  const auto wrapj = [&](int j) { return j < 0 ? j + ny : j >= ny ? j - ny : j; };
+  // swept column c of a colour: region coordinates
+  const auto ycol = [](int c) { return 1 + c / (kMgReg / 2 - 1); };
+  const auto xcol = [&](int c, int y, int color) { return 1 + 2 * (c % (kMgReg / 2 - 1)) + ((1 + y + color) & 1); };
+  double r[2][NR];
+#pragma unroll
+  for (int color = 0; color < 2; color++)
+#pragma unroll
+    for (int u = 0; u < NR; u++) {
+      const int q = tid + u * TH, k = min(q / kMgHalf, nz - 1), c = q % kMgHalf, y = ycol(c);
+      r[color][u] = L.rhs[wrapi(i0 + xcol(c, y, color)) + (long)wrapj(j0 + y) * nx + k * plane];
+    }
+  {
+    constexpr int NK = 4, H = S / 2;
+    for (int q0 = tid; q0 < H * nz; q0 += TH * NK) {
+      double v[NK];
+#pragma unroll
+      for (int u = 0; u < NK; u++) {
+        const int q = min(q0 + u * TH, H * nz - 1), k = q / H, c = q % H, y = c / (kMgReg / 2);
+        const int i = wrapi(i0 + 2 * (c % (kMgReg / 2)) + ((y + 1) & 1)), j = wrapj(j0 + y);
+        v[u] = L.phi[i + (long)j * nx + k * plane];
+        if (PRO) {
+          const int I = i / 2, J = j / 2, cx = Cs.nx, cy = Cs.ny;
+          const int Ix = (i & 1) ? (I + 1 < cx ? I + 1 : 0) : (I > 0 ? I - 1 : cx - 1);
+          const int Jy = (j & 1) ? (J + 1 < cy ? J + 1 : 0) : (J > 0 ? J - 1 : cy - 1);
+          const double *E = Cs.phi + (long)k * cx * cy;
+          const double c00 = E[I + (long)J * cx], c10 = E[Ix + (long)J * cx];
+          const double c01 = E[I + (long)Jy * cx], c11 = E[Ix + (long)Jy * cx];
+          const double ex0 = 0.75 * c00 + 0.25 * c10, ex1 = 0.75 * c01 + 0.25 * c11;
+          v[u] = v[u] + (0.75 * ex0 + 0.25 * ex1);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < NK; u++) {
+        const int q = q0 + u * TH, k = q / H, c = q % H, y = c / (kMgReg / 2);
+        if (q < H * nz) hs[k * S + y * kMgReg + 2 * (c % (kMgReg / 2)) + ((y + 1) & 1)] = v[u];
+      }
+    }
+    mg_tab_fill<TH>(tb, az, den, e, nz, np);
+  }
+#pragma unroll 1
+  for (int s = 0; s < 2; s++)
+#pragma unroll
+  for (int color = 0; color < 2; color++) {
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < NR; u++) {
+      const int q = tid + u * TH, k = q / kMgHalf, c = q % kMgHalf, y = ycol(c);
+      if (k < np) {
+        double *x = hs + k * S + y * kMgReg + xcol(c, y, color);
+        const double hv = L.ax * (x[-1] + x[1]) + L.ay * (x[-kMgReg] + x[kMgReg]);
+        *x = k < nz ? hv - r[color][u] : 1.0;
+      }
+    }
+    __syncthreads();
+    if (tid < kMgHalf) mg_column<S>(hs + ycol(tid) * kMgReg + xcol(tid, ycol(tid), color), tb, nz, np);
+  }
+  __syncthreads();
+  for (int q = tid; q < kMgTile * kMgTile * nz; q += TH) {
+    const int k = q / (kMgTile * kMgTile), c = q % (kMgTile * kMgTile), y = 4 + c / kMgTile, x = 4 + c % kMgTile;
+    L.phi2[(i0 + x) + (long)(j0 + y) * nx + k * plane] = hs[k * S + y * kMgReg + x];
   }
 }
 
@@ -420,9 +573,35 @@ void launch_mg_zero(double *a, long n, hipStream_t st) {
 void launch_mg_sweep(const MgLevel &L, const double *az, const double *den, const double *e, int color,
                      hipStream_t st) {
   const long cols = (long)(L.nx / 2) * L.ny;
-  const size_t sh = (size_t)mg_pad(L.nz) * (kMgCols + 3) * sizeof(double);
+  const size_t sh = (size_t)mg_pad(L.nz) * (kMgCols + 4) * sizeof(double);
   if (sh > 65536) (void)lds_limit_raise((const void *)k_mg_sweep, sh);
   hipLaunchKernelGGL(k_mg_sweep, dim3(nblk(cols, kMgCols)), dim3(kMgThreads), sh, st, L, az, den, e, color);
+}
+
+// A smoothing of level L from phi to phi2; coarse: the level whose correction
+// is added first (or null).
+bool mg_smooth_wanted(const MgLevel &L) {
+  return 2 * mg_smooth_lds(L.nz) <= 160 * 1024 && (long)L.nx * L.ny / (kMgTile * kMgTile) <= kMgSmoothMaxTiles;
+}
+
+void launch_mg_smooth(const MgLevel &L, const MgLevel *coarse, const double *az, const double *den, const double *e,
+                      hipStream_t st) {
+  const size_t sh = mg_smooth_lds(L.nz);
+  const MgLevel Cs = coarse ? *coarse : MgLevel{};
+  const auto run = [&](auto nr, auto pro) {
+    constexpr int NR = decltype(nr)::value;
+    constexpr bool PRO = decltype(pro)::value;
+    if (sh > 65536) (void)lds_limit_raise((const void *)k_mg_smooth<NR, PRO>, sh);
+    hipLaunchKernelGGL((k_mg_smooth<NR, PRO>), dim3(L.nx * L.ny / (kMgTile * kMgTile)), dim3(kMgSmoothThreads), sh, st,
+                       L, Cs, az, den, e);
+  };
+  // values of a colour: swept columns times padded levels, over the threads
+  const int need = (kMgHalf * mg_pad(L.nz) + kMgSmoothThreads - 1) / kMgSmoothThreads;
+  const auto pro = [&](auto nr) { coarse ? run(nr, std::true_type{}) : run(nr, std::false_type{}); };
+  if (need <= 4)
+    pro(std::integral_constant<int, 4>{});
+  else
+    pro(std::integral_constant<int, kMgMaxNr>{});
 }
 
 int mg_resmax_blocks(const MgLevel &L) { return (int)nblk((long)L.nx * L.ny * L.nz, 256); }

@@ -121,6 +121,7 @@ struct MgLevel {
   int nx, ny, nz;
   double ax, ay;  // 1/dx^2, 1/dy^2 of the level
   double *phi, *rhs;
+  double *phi2;  // the other array of phi, where smoothings are whole launches (else null)
 };
 // Work arrays and host tables of the exact coarsest-level solve.
 struct MgCoarse {
@@ -136,6 +137,9 @@ void launch_mg_to_phi(const Geo &g, const double *phi0, double *Phi, hipStream_t
 void launch_mg_zero(double *a, long n, hipStream_t st);
 void launch_mg_sweep(const MgLevel &L, const double *az, const double *den, const double *e, int color,
                      hipStream_t st);
+bool mg_smooth_wanted(const MgLevel &L);
+void launch_mg_smooth(const MgLevel &L, const MgLevel *coarse, const double *az, const double *den, const double *e,
+                      hipStream_t st);
 int mg_resmax_blocks(const MgLevel &L);
 void launch_mg_resmax(const MgLevel &L, const double *az, const double *cz, double *partial, hipStream_t st);
 void launch_mg_restrict(const MgLevel &F, const MgLevel &Cs, const double *az, const double *cz, hipStream_t st);

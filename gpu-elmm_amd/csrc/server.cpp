@@ -155,9 +155,10 @@ int elmm_footprint(const elmm_config *cfg, int64_t *bytes) {
   const int nslots = cfg->nscalars + (cfg->enable_buoyancy ? 1 : 0) + (cfg->enable_moisture ? 1 : 0);
   int64_t b = (int64_t)ntot * (12 * e + 3 * e * nslots + 3 * 8 + 7 + 4 + 1);
   if (cfg->poisson_solver == ELMM_POISSON_MG) {
-    // multigrid: phi and rhs per level (x and y halved: at most 4/3 of the
-    // cells) and the coarsest level's work arrays (below one level 0 array)
-    b += (int64_t)cfg->nx * cfg->ny * cfg->nz * 2 * 8 * 4 / 3 + (int64_t)cfg->nx * cfg->ny * cfg->nz * 8;
+    // multigrid: phi, its other array and rhs per level (x and y halved: at
+    // most 4/3 of the cells) and the coarsest level's work arrays (below one
+    // level 0 array)
+    b += (int64_t)cfg->nx * cfg->ny * cfg->nz * 3 * 8 * 4 / 3 + (int64_t)cfg->nx * cfg->ny * cfg->nz * 8;
   } else {
     // spectral array: complex FP32 with refinement sweeps, complex FP64 otherwise
     b += (int64_t)Mp * cfg->ny * cfg->nz * 2 * es;

@@ -49,12 +49,20 @@ def test_z_solve_lengths(require_gpu, nx, ny, nz):
     _same(*_run(cfg), cfg)
 
 
-# the line sweep stages columns in groups of 8 layers and 16 modes; stretched z
-@pytest.mark.parametrize("nx,ny,nz", [(12, 20, 9), (36, 8, 22), (16, 16, 15)])
-def test_multigrid_column_lengths(require_gpu, nx, ny, nz):
-    cfg = cases.channel_config(nx, ny, nz, poisson_solver=capi.POISSON_MG)
+# the line sweep takes levels in groups of 4 and 16 columns a block, the whole
+# smoothing 4x4 columns with wrapped rings up to 68 levels and 512 tiles; the
+# coarsest solve in LDS and beyond it; stretched z.  still: a flow at rest but
+# for a few cells, whose columns hold zeros (quotients that the sweep divides)
+@pytest.mark.parametrize("still", [False, True])
+@pytest.mark.parametrize("nx,ny,nz", [(12, 20, 9), (36, 8, 22), (16, 16, 15), (8, 8, 5), (40, 24, 68), (64, 16, 69),
+                                      (144, 96, 6), (36, 36, 10)])
+def test_multigrid_column_lengths(require_gpu, nx, ny, nz, still):
+    cfg = cases.channel_config(nx, ny, nz, poisson_solver=capi.POISSON_MG, mg_cycles_max=3)
     case = capi.Case(cfg)
     f = cases.channel_fields(cfg, seed=4)
+    if still:
+        f = tuple(np.zeros_like(a) for a in f[:4]) + ([],)
+        f[0][5:7, 4:6, 4:6] = 0.25
     o, s = Oracle(cfg, case), capi.Solver(cfg, case)
     for x in (o, s):
         cases.upload_initial(x, cfg, f)
