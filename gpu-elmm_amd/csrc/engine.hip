@@ -1336,7 +1336,7 @@ void Engine<T>::setup_lists(const elmm_lists &L) {
       upload_vec(wmp_qflux, qf);
     }
     // point sources, then (with buoyancy) one slot per wall-model point for
-    // the temperature's wall source written by k_wm_ustar every stage
+    // the temperature's wall source written by k_surface every stage
     src_n = L.src_n;
     std::vector<double> sflux(L.src_flux, L.src_flux + L.src_n);
     if (tslot >= 0) sflux.resize(src_n + (mslot >= 0 ? 2 : 1) * (size_t)wmp_n, 0.0);

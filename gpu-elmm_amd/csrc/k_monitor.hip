@@ -1,11 +1,9 @@
-// k_monitor.hip - per-step diagnostics kept in device memory: the CFL
-// number of TimeStepLength with the divergence test of the main loop, the
-// standalone CFL scan of variable time steps, and TMarchRK3's delta.
+// k_monitor.hip - TMarchRK3's delta, kept in device memory (the CFL number and
+// the divergence test of a step are part of k_surface).
 //
-// Every kernel reads and writes the handle's StepMon record only, with
-// launch arguments that are constant for a configuration, so the kernels can
-// sit inside captured step graphs; the host reads the record after a
-// synchronisation.
+// The kernels read and write the handle's StepMon record only, with launch
+// arguments that are constant for a configuration, so they can sit inside
+// captured step graphs; the host reads the record after a synchronisation.
 #include <cmath>
 
 #include "device_common.hpp"
@@ -28,11 +26,6 @@ __device__ inline double block_reduce(double v, Op op) {
     for (int w = 1; w < 4; w++) s = op(s, red[w]);
   __syncthreads();
   return s;
-}
-
-__device__ inline double nan_max(double a, double b) {
-  if (a != a || b != b) return INFINITY;
-  return a > b ? a : b;
 }
 
 }  // namespace
