@@ -2033,7 +2033,8 @@ void Engine<T>::stage(int st, bool last) {
     }
   }
   // BoundUVW of the new velocity: nothing before the projection reads its
-  // ghost cells (the divergence wraps its indices, IB taps are interior)
+  // ghost cells (the divergence wraps its x and y indices and takes W as 0 on
+  // the walls, IB taps are interior)
   const bool use_q = cfg.ib_mass_sources && has_ib();
   if (has_ib()) {
     if (!ib_interior) bound_uvw(u2, v2, w2);

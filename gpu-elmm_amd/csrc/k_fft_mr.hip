@@ -276,10 +276,11 @@ __global__ void __launch_bounds__(kMrThreads)
       } else if (MODE == kMrIn) {
         r[c] = rhs_in[p];
       } else {
-        // U(0) and V(0) by index wrap, as in k_fft_x_fwd
+        // U(0) and V(0) by index wrap, W = 0 on the walls, as in k_fft_x_fwd
         const double du = (double)U[p] - (double)U[i > 0 ? p - 1 : p - 1 + g.nx];
         const double dv = (double)V[p] - (double)V[j > 1 ? p - g.sy : p - g.sy + (long)g.ny * g.sy];
-        const double dw = (double)W[p] - (double)W[p - g.sz];
+        const double wt = (double)W[p], wb = (double)W[p - g.sz];
+        const double dw = (k < g.nz ? wt : 0.0) - (k > 1 ? wb : 0.0);
         r[c] = div_rn(du, g.dxmin, g.rdx) + div_rn(dv, g.dymin, g.rdy) +
                (g.variable_z ? dw / g.dzPr[k] : div_rn(dw, g.dzmin, g.rdz));
       }

@@ -67,10 +67,12 @@ __global__ void __launch_bounds__(256) k_mg_rhs(Geo g, const T *__restrict__ U, 
   const int i = (int)(t % g.nx) + 1, j = (int)((t / g.nx) % g.ny) + 1, k = (int)(t / ((long)g.nx * g.ny)) + 1;
   const long p = gix(g, i, j, k);
   const double dz = g.variable_z ? g.dzPr[k] : g.dzmin;
-  // U(0) and V(0) by index wrap (periodic x and y)
+  // U(0) and V(0) by index wrap (periodic x and y), W = 0 on the walls (see
+  // k_fft_x_fwd)
   const long pw = i > 1 ? p - 1 : p - 1 + g.nx, ps = j > 1 ? p - g.sy : p - g.sy + (long)g.ny * g.sy;
+  const double wt = (double)W[p], wb = (double)W[p - g.sz];
   double r = ((double)U[p] - (double)U[pw]) / g.dxmin + ((double)V[p] - (double)V[ps]) / g.dymin +
-             ((double)W[p] - (double)W[p - g.sz]) / dz;
+             ((k < g.nz ? wt : 0.0) - (k > 1 ? wb : 0.0)) / dz;
   if (Q) r = r - Q[p];
   r = r * dt2_rec;
   rhs0[t] = r;

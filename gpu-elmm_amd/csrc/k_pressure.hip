@@ -224,12 +224,15 @@ __global__ void __launch_bounds__(kFftThreads)
     } else if constexpr (MODE == kRhsIn) {
       return rhs_in[p];
     } else {
-      // U(0) and V(0) by index wrap (periodic x and y): the ghost cells of the
-      // stage's velocity are filled after the projection only; W(0) = 0 of
-      // the wall is in the field
+      // U(0) and V(0) by index wrap (periodic x and y), W = 0 on the walls by
+      // selection: the ghost cells of the stage's velocity are filled after
+      // the projection only, and until then hold what the array's earlier use
+      // as the current field left there (an uploaded W may be non-zero on its
+      // wall faces 0 and nz)
       const double du = (double)U[p] - (double)U[m > 0 ? p - 1 : p - 1 + g.nx];
       const double dv = (double)V[p] - (double)V[(row & (pp.ny - 1)) > 0 ? p - g.sy : p - g.sy + (long)g.ny * g.sy];
-      const double dw = (double)W[p] - (double)W[p - g.sz];
+      const double wt = (double)W[p], wb = (double)W[p - g.sz];
+      const double dw = (k < g.nz ? wt : 0.0) - (k > 1 ? wb : 0.0);
       if constexpr ((MODE & kRhsFast) != 0)
         return div_rn_nz(du, g.dxmin, g.rdx) + div_rn_nz(dv, g.dymin, g.rdy) + div_rn_nz(dw, g.dzmin, g.rdz);
       else

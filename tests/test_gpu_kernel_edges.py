@@ -101,6 +101,25 @@ def test_ghosts_are_images(require_gpu, nx, ny, nz):
         np.testing.assert_array_equal(a, o.download(c))
 
 
+# W uploaded between steps with values on its wall faces and in all its ghost
+# cells (a restart, nudging): the first stage reads them as they are, the
+# later ones must not find them again.  Power-of-two, mixed-radix and
+# multigrid right-hand sides; the box -2..n+3 holds both faces, 1..n face nz
+@pytest.mark.parametrize("solids", [False, True])
+@pytest.mark.parametrize("lb", [-2, 1])
+@pytest.mark.parametrize("nx,ny,nz,mg", [(16, 8, 6, False), (12, 18, 7, False), (20, 12, 6, True)])
+def test_w_uploaded_between_steps(require_gpu, nx, ny, nz, mg, lb, solids):
+    kw = dict(poisson_solver=capi.POISSON_MG, mg_cycles_max=3) if mg else {}
+    cfg = cases.uniform_config(nx, ny, nz, dx=1.0, dt=0.02, **kw)
+    o, s = _run(cfg, cuboids=[(4.0, 8.0, 2.0, 6.0, 0.0, 2.2)] if solids else ())
+    n = np.array(capi.ghosted_shape(cfg)) - (0 if lb == -2 else 6)
+    w = np.random.default_rng(11).uniform(-0.3, 0.3, n)
+    for x in (o, s):
+        x.upload(capi.F_W, w, lb=lb)
+        x.step(2)
+    _same(o, s, cfg)
+
+
 # boxes of a field: inside it, exactly it, beyond it; fields of less than a
 # slot, of one row per slab and of several slots per thread
 @pytest.mark.parametrize("n", [(6, 4, 4), (48, 24, 20), (192, 144, 96)])
