@@ -100,10 +100,14 @@ __global__ void __launch_bounds__(256) k_mg_zero(double *__restrict__ a, long n)
 // LDS for the two passes, and writes them back.  (One thread per column
 // loading as it went: 30 us a sweep of 128x64 columns of 64 levels, bound by
 // a memory round trip per four levels; staged about 9.)
-// Levels are padded to whole groups of ZB, so the chain carries no conditions and a group's operands are
-// fetched while the previous group is worked through.
+// Levels are padded to whole groups of ZB, so the chain carries no conditions
+// and a group's operands are fetched while the previous group is worked
+// through.
 constexpr int kMgCols = 16, kMgThreads = 256, ZB = 4;
 __host__ __device__ constexpr int mg_pad(int nz) { return (nz + ZB - 1) / ZB * ZB; }
+// the columns of a block and the tables of MgTab: up to 1024 levels fit a CU
+constexpr size_t mg_sweep_lds(int nz) { return (size_t)mg_pad(nz) * (kMgCols + 4) * sizeof(double); }
+static_assert(mg_sweep_lds(1024) <= 160 * 1024 && mg_sweep_lds(1025) > 160 * 1024, "k_mg_sweep's tallest column");
 // Tables of a sweep in LDS: az, den, RN(1/den) and e of each level.
 struct MgTab {
   double *az, *den, *rden, *e;
@@ -254,6 +258,41 @@ __global__ void __launch_bounds__(kMgThreads) k_mg_sweep(MgLevel L, const double
   if (t < ncol) {
 #pragma unroll 4
     for (int k = threadIdx.x / kMgCols; k < nz; k += kMgThreads / kMgCols) P[c + (long)k * plane] = hs[k * kMgCols + l];
+  }
+}
+
+// The sweep of columns too tall for LDS, any number of levels: one thread per
+// column, the forward values stored in place.  Same operations as
+// k_mg_sweep, whose quotients are the divisions' bits.
+__global__ void __launch_bounds__(256) k_mg_sweep_tall(MgLevel L, const double *__restrict__ az,
+                                                       const double *__restrict__ den, const double *__restrict__ e,
+                                                       int color) {
+  const int half = L.nx / 2;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= half * L.ny) return;
+  const int j = t / half + 1, ii = t - (j - 1) * half;
+  const int i = 2 * ii + (((j + color) & 1) ? 1 : 2);
+  const int nx = L.nx, nz = L.nz;
+  const long plane = (long)nx * L.ny;
+  const long c = (i - 1) + (long)(j - 1) * nx;
+  const long w = (wrap_lo(i, nx) - 1) + (long)(j - 1) * nx, ea = (wrap_hi(i, nx) - 1) + (long)(j - 1) * nx;
+  const long so = (i - 1) + (long)(wrap_lo(j, L.ny) - 1) * nx, no = (i - 1) + (long)(wrap_hi(j, L.ny) - 1) * nx;
+  double *P = L.phi;
+  const double *R = L.rhs;
+  double gv = 0;
+#pragma unroll 4
+  for (int k = 1; k <= nz; k++) {
+    const long o = (long)(k - 1) * plane;
+    const double h = L.ax * (P[w + o] + P[ea + o]) + L.ay * (P[so + o] + P[no + o]);
+    gv = ((h - R[c + o]) + az[k - 1] * gv) / den[k - 1];
+    P[c + o] = gv;
+  }
+  double x = gv;
+#pragma unroll 4
+  for (int k = nz - 1; k >= 1; k--) {
+    const long o = (long)(k - 1) * plane;
+    x = P[c + o] + e[k - 1] * x;
+    P[c + o] = x;
   }
 }
 
@@ -575,7 +614,11 @@ void launch_mg_zero(double *a, long n, hipStream_t st) {
 void launch_mg_sweep(const MgLevel &L, const double *az, const double *den, const double *e, int color,
                      hipStream_t st) {
   const long cols = (long)(L.nx / 2) * L.ny;
-  const size_t sh = (size_t)mg_pad(L.nz) * (kMgCols + 4) * sizeof(double);
+  const size_t sh = mg_sweep_lds(L.nz);
+  if (sh > 160 * 1024) {
+    hipLaunchKernelGGL(k_mg_sweep_tall, dim3(nblk(cols, 256)), dim3(256), 0, st, L, az, den, e, color);
+    return;
+  }
   if (sh > 65536) (void)lds_limit_raise((const void *)k_mg_sweep, sh);
   hipLaunchKernelGGL(k_mg_sweep, dim3(nblk(cols, kMgCols)), dim3(kMgThreads), sh, st, L, az, den, e, color);
 }

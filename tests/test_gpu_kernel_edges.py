@@ -71,6 +71,14 @@ def test_multigrid_column_lengths(require_gpu, nx, ny, nz, still):
     _same(o, s, cfg)
 
 
+# the tallest column that the line sweep holds in LDS and taller ones, which
+# it sweeps in global memory
+@pytest.mark.parametrize("nx,ny,nz", [(8, 8, 1024), (8, 8, 1025), (12, 8, 1100)])
+def test_multigrid_tall_columns(require_gpu, nx, ny, nz):
+    cfg = cases.uniform_config(nx, ny, nz, dx=1.0, dt=0.02, poisson_solver=capi.POISSON_MG, mg_cycles_max=2)
+    _same(*_run(cfg, steps=1), cfg)
+
+
 # walk lengths and tiles of the z-marching kernels: layers that no walk
 # divides, rows and columns that leave tiles partly empty, two scalars
 @pytest.mark.parametrize("nx,ny,nz", [(64, 8, 5), (66, 10, 17), (128, 12, 31), (36, 64, 65)])
