@@ -1553,23 +1553,23 @@ void Engine<T>::setup_lists(const elmm_lists &L) {
       upload_vec(qmask, qm);
     }
     for (int c = 0; c < 3; c++) {
-      null_n[c] = L.null_n[c];
-      std::vector<int32_t> v(L.null_ijk[c], L.null_ijk[c] + 3 * (size_t)null_n[c]);
-      // and the x and y ghost cells that hold their images, which the
-      // projection has written by then
+      // the interior points and the x and y ghost cells that hold their
+      // images, which the projection has written by then (a point in a ghost
+      // cell takes its interior source's value from BoundUVW, null or not)
+      std::vector<int32_t> v;
       const int n[2] = {cfg.nx, cfg.ny};
       for (int p = 0; p < L.null_n[c]; p++) {
-        const int q[3] = {v[3 * (size_t)p], v[3 * (size_t)p + 1], v[3 * (size_t)p + 2]};
+        const int32_t *q = &L.null_ijk[c][3 * (size_t)p];
+        if (q[0] < 1 || q[0] > g.n[c][0] || q[1] < 1 || q[1] > g.n[c][1] || q[2] < 1 || q[2] > g.n[c][2]) continue;
         int im[2][3], ni[2];
         for (int a = 0; a < 2; a++) {
           ni[a] = 0;
           im[a][ni[a]++] = q[a];
-          if (q[a] >= 1 && q[a] <= 3) im[a][ni[a]++] = q[a] + n[a];
-          if (q[a] > n[a] - 3 && q[a] <= n[a]) im[a][ni[a]++] = q[a] - n[a];
+          if (q[a] <= 3) im[a][ni[a]++] = q[a] + n[a];
+          if (q[a] > n[a] - 3) im[a][ni[a]++] = q[a] - n[a];
         }
         for (int b = 0; b < ni[1]; b++)
-          for (int a = 0; a < ni[0]; a++)
-            if (a || b) v.insert(v.end(), {im[0][a], im[1][b], q[2]});
+          for (int a = 0; a < ni[0]; a++) v.insert(v.end(), {im[0][a], im[1][b], q[2]});
       }
       null_n[c] = (int)(v.size() / 3);
       upload_vec(null_ijk[c], v);

@@ -4,6 +4,8 @@ src/tsteps.f90:368-418) and a ScalFl viscosity list whose points read earlier
 points' targets (serial loop, src/dynamics.f90:899-902, which the device
 runs in dependency levels).  Bit-identical to the oracle after 1 and 3
 steps, in the FP64 form."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -78,3 +80,37 @@ def test_gpu_wm_ustar_matches_oracle(require_gpu, channel):
         assert rel <= 1e-5, rel
     for x in (o, s, s32):
         x.close()
+
+
+def _null_case(case, comp, ijk):
+    """A copy of a case's list view with the nullified points of one component
+    replaced."""
+    c = ListsCase(case, 3, *case.ib_list(3))
+    pts = np.ascontiguousarray(ijk, dtype=np.int32)
+    c._keep.append(pts)
+    c.view.null_n[comp] = len(pts)
+    c.view.null_ijk[comp] = pts.ctypes.data_as(C.POINTER(C.c_int32))
+    return c
+
+
+def _same_after_steps(cfg, lc):
+    f = cases.initial_fields(cfg, u0=1.5, amp=0.2, seed=9)
+    o, s = Oracle(cfg, lc), capi.Solver(cfg, lc)
+    for x in (o, s):
+        cases.upload_initial(x, cfg, f)
+        x.init()
+        x.step(2)
+    err = compare_state(s, o, cfg)
+    for c in range(3):  # the ghost cells too
+        err[f"whole {c}"] = float(np.abs(s.download(c) - o.download(c)).max())
+    print(err, flush=True)
+    assert max(err.values()) == 0.0, err
+
+
+@pytest.mark.parametrize("comp", [0, 1, 2])
+def test_gpu_nullified_points_in_ghost_cells(require_gpu, comp):
+    """NullInterior (src/tsteps.f90:543-567) zeroes its points as listed and
+    BoundUVW follows, so a point in a ghost cell takes its source's value."""
+    cfg = cases.uniform_config(16, 8, 6, dx=1.0, dt=0.05)
+    pts = [(4, 4, 2), (1, 8, 3), (0, 3, 2), (17, 5, 3), (-2, -1, 2), (5, 0, 4), (6, 9, 1), (7, 3, 0), (8, 3, 7)]
+    _same_after_steps(cfg, _null_case(capi.Case(cfg), comp, pts))
