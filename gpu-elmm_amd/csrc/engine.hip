@@ -2037,8 +2037,10 @@ void Engine<T>::stage(int st, bool last) {
   // the walls, IB taps are interior)
   const bool use_q = cfg.ib_mass_sources && has_ib();
   if (has_ib()) {
+    // with points or taps in ghost cells, which interpolation and mass sources
+    // read, the fills before and after it as the reference has them
     if (!ib_interior) bound_uvw(u2, v2, w2);
-    ib_momentum(u2, v2, w2, false);
+    ib_momentum(u2, v2, w2, !ib_interior);
   }
   if (use_q) timed(ELMM_T_IB, [&] { launch_mass_sources(g, q_terms.view(), u2, v2, w2, Q.as<double>(), stream); });
   pressure_correction(u2, v2, w2, use_q, sc.coef, last && want_diag, true);

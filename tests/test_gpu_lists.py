@@ -114,3 +114,22 @@ def test_gpu_nullified_points_in_ghost_cells(require_gpu, comp):
     cfg = cases.uniform_config(16, 8, 6, dx=1.0, dt=0.05)
     pts = [(4, 4, 2), (1, 8, 3), (0, 3, 2), (17, 5, 3), (-2, -1, 2), (5, 0, 4), (6, 9, 1), (7, 3, 0), (8, 3, 7)]
     _same_after_steps(cfg, _null_case(capi.Case(cfg), comp, pts))
+
+
+@pytest.mark.parametrize("inside", [False, True])
+@pytest.mark.parametrize("use_q", [0, 1])
+def test_gpu_ib_points_and_taps_in_ghost_cells(require_gpu, use_q, inside):
+    """Points in ghost cells (IBMomentum, src/tsteps.f90:368-418, then
+    BoundUVW: the ghost takes its source's value) and taps in ghost cells, W's
+    wall face among them; the mass sources read the points after BoundUVW.
+    inside: only the taps are in ghost cells."""
+    cfg = cases.uniform_config(16, 8, 6, dx=1.0, dt=0.05, ib_mass_sources=use_q)
+    case = capi.Case(cfg)
+    for comp, tgt in ((0, [(0, 4, 2), (5, 4, 2), (18, 3, 3)]), (1, [(4, 0, 2), (4, 8, 2), (6, 9, 3)]),
+                      (2, [(0, 3, 2), (4, 4, 1), (4, 9, 3)])):
+        if inside:
+            tgt = [(min(max(i, 1), 16), min(max(j, 1), 8), k) for i, j, k in tgt]
+        src = [(1, 4, 2), (2, 4, 2), (5, 4, 3), (5, 4, 0), (17, 3, 3), (16, -1, 3)]
+        case = ListsCase(case, comp, np.array(tgt), np.array([0, 2, 4, 6]), np.array(src),
+                         np.array([0.7, 0.2, 0.6, 0.3, 0.5, -0.4]))
+    _same_after_steps(cfg, case)
