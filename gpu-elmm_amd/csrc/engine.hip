@@ -120,12 +120,28 @@ int current_device() {
 }
 void use_device(int d) { (void)hipSetDevice(d); }
 
+namespace {
+// Makes device d current on this thread for the scope.
+struct DeviceScope {
+  explicit DeviceScope(int d) {
+    HIPCHK(hipGetDevice(&prev));
+    HIPCHK(hipSetDevice(d));
+  }
+  ~DeviceScope() { (void)hipSetDevice(prev); }
+  DeviceScope(const DeviceScope &) = delete;
+  DeviceScope &operator=(const DeviceScope &) = delete;
+  int prev = 0;
+};
+}  // namespace
+
 // Pinned host slots of the field transfers, shared by the handles of the
 // process: at most kKeep (64 MiB) stay allocated between transfers, and the
 // last handle to go gives them back.  A transfer holds its slots alone; the
 // events are created with the slots (pinned memory and events cost
 // milliseconds to create, a transfer of a small field tens of microseconds).
-// Callers hold a HostOpLock (the allocations and frees are host operations).
+// Callers hold a HostOpLock (the allocations and frees are host operations),
+// and the device of the stream that the events are recorded on is current
+// where Slots are made.
 class PinnedPool {
  public:
   static constexpr size_t kSlotBytes = 2 << 20, kKeep = 32;
@@ -1702,6 +1718,7 @@ void Engine<T>::xfer(int field, int lb, const int32_t ext[3], double *host, bool
   }
   if (!d) throw ArgError("unknown field id " + std::to_string(field));
   if (ext[0] <= 0 || ext[1] <= 0 || ext[2] <= 0) throw ArgError("extents must be positive");
+  const DeviceScope scope(device);  // the caller may have another device current
   const int n[3] = {cfg.nx, cfg.ny, cfg.nz};
   int lo[3], hi[3];
   for (int a = 0; a < 3; a++) {
