@@ -2195,7 +2195,11 @@ void Engine<T>::autotune() {
   const auto key = std::make_tuple((int)sizeof(T), cfg.nx, cfg.ny, cfg.nz, nsc);
   TileChoice c{mom_tile, zchunk, sgs_cap, zchunk_scalar};
   bool hit = false;
-  {
+  // a handle with settings fixed by the environment neither takes another's
+  // choice, which would replace them (and the room for the CFL partials is
+  // sized by its own SGS chunk), nor leaves them to others
+  const bool fixed = env_mom_tile || env_zchunk || env_scalar_zchunk || env_sgs_zchunk;
+  if (!fixed) {
     std::lock_guard<std::mutex> lock(g_tune_mu);
     auto it = g_tune_cache.find(key);
     if (it != g_tune_cache.end()) {
@@ -2304,8 +2308,10 @@ void Engine<T>::autotune() {
       (void)hipEventDestroy(e0);
       (void)hipEventDestroy(e1);
     }
-    std::lock_guard<std::mutex> lock(g_tune_mu);
-    g_tune_cache[key] = c;
+    if (!fixed) {
+      std::lock_guard<std::mutex> lock(g_tune_mu);
+      g_tune_cache[key] = c;
+    }
   }
   mom_tile = c.mom_tile;
   zchunk = c.zchunk;

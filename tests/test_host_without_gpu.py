@@ -1,0 +1,87 @@
+"""Host code of the engine on a stand-in for the HIP runtime
+(hip_standin.cpp), without a GPU: transfers of a handle whose device is not
+the calling thread's current one, and the autotuner's cache beside settings
+fixed by the environment."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes, os, sys
+hip = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)  # found before the HIP runtime itself
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+from elmm_amd import capi, cases
+"""
+
+TRANSFERS = """
+def device():
+    d = ctypes.c_int(-1)
+    hip.hipGetDevice(ctypes.byref(d))
+    return d.value
+
+n = int(sys.argv[3])
+cfg = cases.uniform_config(n, n, n, dx=1.0, dt=0.02, nscalars=1)
+case = capi.Case(cfg)
+solvers = []
+for d in (0, 1):
+    hip.hipSetDevice(d)
+    solvers.append(capi.Solver(cfg, case))
+rng = np.random.default_rng(1)
+for d in (0, 1):
+    hip.hipSetDevice(d)
+    for s in solvers:
+        for field in (capi.F_U, capi.F_SCALAR):
+            a = rng.standard_normal(capi.ghosted_shape(cfg))
+            s.upload(field, a)
+            assert device() == d, "upload changed the caller's device"
+            assert np.array_equal(s.download(field), a)
+            assert device() == d, "download changed the caller's device"
+print("ok")
+"""
+
+TUNED = """
+cfg = cases.uniform_config(64, 64, 256, dx=1.0, dt=0.02, nscalars=1, autotune=1)
+case = capi.Case(cfg)
+
+def tiles(env):
+    if env:
+        os.environ["ELMM_SGS_ZCHUNK"] = env
+    else:
+        os.environ.pop("ELMM_SGS_ZCHUNK", None)
+    s = capi.Solver(cfg, case)
+    s.init()
+    s.step(1, diag=False)
+    return s.tiles()["sgs_zchunk"]
+
+got = [tiles(e) for e in sys.argv[3].split(",")]
+assert all(g == int(e) if e else g in (13, 16, 26, 32) for g, e in zip(got, sys.argv[3].split(","))), got
+print("ok")
+"""
+
+
+def _run(tmp_path, script, arg):
+    lib = str(tmp_path / "libhip_standin.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I", "/opt/rocm/include",
+                    os.path.join(HERE, "hip_standin.cpp"), "-o", lib], check=True)
+    r = subprocess.run([sys.executable, "-c", PRELUDE + script, lib,
+                        os.path.join(os.path.dirname(HERE), "gpu-elmm_amd"), arg],
+                       capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout + r.stderr
+
+
+# one task, on the caller's thread; several, on threads of their own
+@pytest.mark.parametrize("n", [8, 96])
+def test_transfers_of_a_handle_on_another_device(tmp_path, n):
+    _run(tmp_path, TRANSFERS, str(n))
+
+
+# a chunk fixed after a tuned handle, and before one (whose room for the SGS
+# kernel's partials is sized by the chunks that the tuner tries)
+@pytest.mark.parametrize("order", [",4", "4,", "40,,4"])
+def test_tuned_choices_and_fixed_settings_stay_apart(tmp_path, order):
+    _run(tmp_path, TUNED, order)
