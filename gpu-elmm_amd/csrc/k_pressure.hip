@@ -505,11 +505,8 @@ __global__ void __launch_bounds__(64)
 // written once.  Levels are padded to whole groups of ZB with zeros (whose
 // elimination gives zeros), so the chain carries no conditions and a group's
 // operands are fetched while the previous group is worked through.
-// Measured against k_solve_z (us with event overhead): 64^3 38 -> 12,
-// 144x144x72 44 -> 17, 256x128x128 80 -> 37, 256x256x128 92 -> 58, but
-// 512x256x128 105 -> 101 and 512x512x128 155 -> 188 (there k_solve_z streams
-// at 4.8 TB/s and the table adds a third of traffic): used up to 1024
-// wavefronts of modes.  ZL = 16 and 64 are slower (256x128x128: 47 and 49).
+// ZL = 16 and 64 are slower (256x128x128: 47 and 49 us against 37).  Where it
+// is used: z_table_wanted.
 constexpr int ZL = 32, ZB = 8, kZThreads = 256;
 
 __host__ __device__ constexpr int z_pad(int nz) { return (nz + ZB - 1) / ZB * ZB; }
@@ -793,8 +790,21 @@ void launch_fft_y(const PoissonPlan<R> &pp, int inverse, hipStream_t st) {
   });
 }
 
+// The table up to 1024 wavefronts of modes, fewer where tall columns leave a
+// CU fewer blocks: with one (nz > 192) or two (nz > 128) the chip works
+// through its blocks in rounds of loads, sweep and stores that hide nothing of
+// each other, while k_solve_z streams and its divisions hide behind the other
+// wavefronts.  us, table / k_solve_z in FP64:
+//   blocks a CU  wavefronts 263 (or 387)  516          734          976
+//   6 (nz 64)    24.3 / 43.7              32.7 / 48.8  40.2 / 52.2  51.2 / 54.8
+//   3 (nz 128)   36.2 / 84.0              56.9 / 95.0  73.2 / 98.5  94.9 / 104.1
+//   2 (nz 192)   89.5 / 133.0 (387)       112 / 140    136 / 144    179 / 151
+//   1 (nz 256)   120 / 169                218 / 186    292 / 191
+// (with FP32 spectra 138 / 136 at 2 and 734).  368 wavefronts at one block a
+// CU 159 / 177, 464 198 / 180; 580 at two 115 / 141.
 bool z_table_wanted(int Mp, int ny, int nz) {
-  return ((long)Mp * ny + 63) / 64 <= 1024 && solve_z_table_lds(nz) <= 160 * 1024;
+  const long waves = ((long)Mp * ny + 63) / 64, percu = 160 * 1024 / (long)solve_z_table_lds(nz);
+  return waves <= std::min(1024L, 340 * percu);
 }
 
 void launch_z_pivots(int nz, int ny, int M, int Mp, const double *lamx, const double *lamy, const double *az,

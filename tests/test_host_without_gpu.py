@@ -2,11 +2,14 @@
 (hip_standin.cpp), without a GPU: transfers of a handle whose device is not
 the calling thread's current one, and the autotuner's cache beside settings
 fixed by the environment."""
+import ctypes as C
 import os
 import subprocess
 import sys
 
 import pytest
+
+from elmm_amd import capi
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 
@@ -85,3 +88,15 @@ def test_transfers_of_a_handle_on_another_device(tmp_path, n):
 @pytest.mark.parametrize("order", [",4", "4,", "40,,4"])
 def test_tuned_choices_and_fixed_settings_stay_apart(tmp_path, order):
     _run(tmp_path, TUNED, order)
+
+
+# the z solve's table of pivots is used where it is the faster solve: not where
+# its columns leave a CU few blocks and the grid has many modes, nor beyond a
+# CU's LDS (arguments: modes a row, rows, levels)
+@pytest.mark.parametrize("modes,used", [((40, 64, 64), 1), ((40, 64, 392), 1), ((40, 64, 400), 0),
+                                        ((136, 256, 192), 1), ((136, 256, 200), 0), ((200, 256, 128), 1),
+                                        ((200, 256, 136), 0), ((264, 512, 64), 0)])
+def test_pivot_table_where_it_is_faster(modes, used):
+    wanted = capi.load()._ZN4elmm14z_table_wantedEiii
+    wanted.argtypes, wanted.restype = [C.c_int] * 3, C.c_bool
+    assert wanted(*modes) == bool(used)
