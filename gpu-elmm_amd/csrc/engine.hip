@@ -1765,7 +1765,6 @@ void Engine<T>::xfer_rows(E *d, const int lo[3], const int hi[3], int lb, const 
   const long nslab = (r1 - r0 + slab - 1) / slab;
   const int w = hi[0] - lo[0] + 1;
   const long hy = ext[0], hz = (long)ext[0] * ext[1];
-  PinnedPool::Slots slots(2 * nth, (size_t)row_bytes);
   auto convert = [&](E *buf, long s) {
     const long b = r0 + s * slab, e = std::min(r1, b + slab);
     if (whole) std::memset(buf, 0, (size_t)((e - b) * row_bytes));
@@ -1780,16 +1779,34 @@ void Engine<T>::xfer_rows(E *d, const int lo[3], const int hi[3], int lb, const 
         for (int i = 0; i < w; i++) h[i] = (double)f[i];
     }
   };
+  // Small spans go through a pageable image in one copy each way: below some
+  // 400 KiB the slots' events and the pins cost more than the copy engine
+  // gives (16^3 FP64 16 against 21 us a field, 24^3 FP32 19 against 24, equal
+  // at 36^3 FP32 of 440 KiB, 32^3 FP64 of 720 KiB 54 against 47)
+  const size_t span = (size_t)((r1 - r0) * row_bytes);
+  if (span <= 400 * 1024) {
+    std::unique_ptr<E[]> image(new E[span / sizeof(E)]);
+    E *dev = d + r0 * g.sy;
+    if (!whole) HIPCHK(hipMemcpy(image.get(), dev, span, hipMemcpyDeviceToHost));
+    convert(image.get(), 0);
+    if (up) HIPCHK(hipMemcpy(dev, image.get(), span, hipMemcpyHostToDevice));
+    return;
+  }
+  // two slots a thread, or the one it uses (a slot that is not in the pool
+  // takes 0.6 ms to pin and 0.4 to free)
+  const int per = nslab > nth ? 2 : 1;
+  PinnedPool::Slots slots(per * nth, (size_t)row_bytes);
   auto task = [&](int t) {
+    if (t >= nslab) return;  // few rows of more than a slot
     HostOpInherit inherit;
     HIPCHK(hipSetDevice(device));
     auto copy = [&](long s, int q, hipMemcpyKind kind) {
       const long b = r0 + s * slab, rows = std::min(r1, b + slab) - b;
-      E *dev = d + b * g.sy, *pin = static_cast<E *>(slots.p[2 * t + q]);
+      E *dev = d + b * g.sy, *pin = static_cast<E *>(slots.p[per * t + q]);
       HIPCHK(hipMemcpyAsync(kind == hipMemcpyDeviceToHost ? (void *)pin : (void *)dev,
                             kind == hipMemcpyDeviceToHost ? (const void *)dev : (const void *)pin,
                             (size_t)(rows * row_bytes), kind, stream));
-      HIPCHK(hipEventRecord(slots.e[2 * t + q], stream));
+      HIPCHK(hipEventRecord(slots.e[per * t + q], stream));
     };
     const bool fetch = !whole;  // the slab's current rows are needed on the host
     int q = 0;
@@ -1798,18 +1815,18 @@ void Engine<T>::xfer_rows(E *d, const int lo[3], const int hi[3], int lb, const 
     for (long s = t; s < nslab; s += nth, q ^= 1) {
       // the other slot: the next slab's rows, once its upload has left it
       if (fetch && s + nth < nslab) {
-        if (busy[q ^ 1]) HIPCHK(hipEventSynchronize(slots.e[2 * t + (q ^ 1)]));
+        if (busy[q ^ 1]) HIPCHK(hipEventSynchronize(slots.e[per * t + (q ^ 1)]));
         copy(s + nth, q ^ 1, hipMemcpyDeviceToHost);
       }
-      if (fetch || busy[q]) HIPCHK(hipEventSynchronize(slots.e[2 * t + q]));
-      convert(static_cast<E *>(slots.p[2 * t + q]), s);
+      if (fetch || busy[q]) HIPCHK(hipEventSynchronize(slots.e[per * t + q]));
+      convert(static_cast<E *>(slots.p[per * t + q]), s);
       if (up) {
         copy(s, q, hipMemcpyHostToDevice);
         busy[q] = true;
       }
     }
     for (int b = 0; b < 2; b++)
-      if (busy[b]) HIPCHK(hipEventSynchronize(slots.e[2 * t + b]));
+      if (busy[b]) HIPCHK(hipEventSynchronize(slots.e[per * t + b]));
   };
   try {
     run_tasks(nth, task);
