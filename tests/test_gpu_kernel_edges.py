@@ -96,7 +96,7 @@ def _periodic_images(a, nx, ny):
 
 # obstacles across the periodic edges: the kernels that write a value there
 # (projection, immersed-boundary points, points inside solids) write its
-# images too; 4 and 5 cells: a cell has images on both sides
+# images too; 4 cells: a cell has images on both sides
 @pytest.mark.parametrize("nx,ny,nz", [(4, 8, 6), (8, 4, 6), (24, 18, 8), (64, 32, 12)])
 def test_ghosts_are_images(require_gpu, nx, ny, nz):
     cfg = cases.uniform_config(nx, ny, nz, dx=1.0, dt=0.02, nscalars=1)
