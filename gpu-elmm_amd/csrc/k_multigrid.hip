@@ -381,20 +381,20 @@ __global__ void __launch_bounds__(kMgSmoothThreads, 4)
 #pragma unroll 1
   for (int s = 0; s < 2; s++)
 #pragma unroll
-  for (int color = 0; color < 2; color++) {
-    __syncthreads();
+    for (int color = 0; color < 2; color++) {
+      __syncthreads();
 #pragma unroll
-    for (int u = 0; u < NR; u++) {
-      const int q = tid + u * TH, k = q / kMgHalf, c = q % kMgHalf, y = ycol(c);
-      if (k < np) {
-        double *x = hs + k * S + y * kMgReg + xcol(c, y, color);
-        const double hv = L.ax * (x[-1] + x[1]) + L.ay * (x[-kMgReg] + x[kMgReg]);
-        *x = k < nz ? hv - r[color][u] : 1.0;
+      for (int u = 0; u < NR; u++) {
+        const int q = tid + u * TH, k = q / kMgHalf, c = q % kMgHalf, y = ycol(c);
+        if (k < np) {
+          double *x = hs + k * S + y * kMgReg + xcol(c, y, color);
+          const double hv = L.ax * (x[-1] + x[1]) + L.ay * (x[-kMgReg] + x[kMgReg]);
+          *x = k < nz ? hv - r[color][u] : 1.0;
+        }
       }
+      __syncthreads();
+      if (tid < kMgHalf) mg_column<S>(hs + ycol(tid) * kMgReg + xcol(tid, ycol(tid), color), tb, nz, np);
     }
-    __syncthreads();
-    if (tid < kMgHalf) mg_column<S>(hs + ycol(tid) * kMgReg + xcol(tid, ycol(tid), color), tb, nz, np);
-  }
   __syncthreads();
   for (int q = tid; q < kMgTile * kMgTile * nz; q += TH) {
     const int k = q / (kMgTile * kMgTile), c = q % (kMgTile * kMgTile), y = 4 + c / kMgTile, x = 4 + c % kMgTile;
