@@ -196,8 +196,10 @@ class PinnedPool {
     void *p;
     hipEvent_t e;
   };
+  // never destroyed: a static object of the program may destroy the last
+  // handle after this library's own static objects have gone
   static std::mutex &mu() {
-    static std::mutex m;
+    static std::mutex &m = *new std::mutex;
     return m;
   }
   static int &users() {
@@ -205,7 +207,7 @@ class PinnedPool {
     return n;
   }
   static std::vector<Free> &pool() {
-    static std::vector<Free> v;
+    static std::vector<Free> &v = *new std::vector<Free>;
     return v;
   }
   static void release(const Free &f) {

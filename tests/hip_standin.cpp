@@ -2,11 +2,15 @@
 // library's host code without a GPU: device memory is host memory, copies
 // happen at once, kernels do nothing.  As in HIP, a stream and an event belong
 // to the device that was current when they were created, and an event can only
-// be recorded on a stream of its own device.
+// be recorded on a stream of its own device.  Freeing host memory that is not
+// allocated ends the program.
 #include <hip/hip_runtime_api.h>
 
+#include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
+#include <set>
 
 namespace {
 thread_local int current = 0;
@@ -14,6 +18,9 @@ struct Owned {
   int device;
 };
 int device_of(hipStream_t s) { return s ? reinterpret_cast<Owned *>(s)->device : current; }
+// never destroyed: used until the process ends
+std::mutex &host_mu = *new std::mutex;
+std::set<void *> &host = *new std::set<void *>;
 alignas(256) double symbol[(1 << 18) + 32];
 }  // namespace
 
@@ -35,8 +42,20 @@ hipError_t hipFree(void *p) {
   std::free(p);
   return hipSuccess;
 }
-hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
-hipError_t hipHostFree(void *p) { return hipFree(p); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+  const hipError_t e = hipMalloc(p, n);
+  std::lock_guard<std::mutex> lock(host_mu);
+  if (e == hipSuccess) host.insert(*p);
+  return e;
+}
+hipError_t hipHostFree(void *p) {
+  std::lock_guard<std::mutex> lock(host_mu);
+  if (!host.erase(p)) {
+    std::fprintf(stderr, "hipHostFree of memory that is not allocated\n");
+    std::_Exit(3);
+  }
+  return hipFree(p);
+}
 hipError_t hipMemset(void *p, int v, size_t n) {
   std::memset(p, v, n);
   return hipSuccess;

@@ -66,6 +66,34 @@ assert all(g == int(e) if e else g in (13, 16, 26, 32) for g, e in zip(got, sys.
 print("ok")
 """
 
+# a handle that a static object of the program destroys, as the process ends
+AT_EXIT = """
+cfg = cases.uniform_config(48, 48, 48, dx=1.0, dt=0.02)
+s = capi.Solver(cfg, capi.Case(cfg))
+s.upload(capi.F_U, np.zeros(capi.ghosted_shape(cfg)))
+owner = ctypes.CDLL(sys.argv[3])
+owner.own.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+owner.own(s._h, ctypes.cast(capi._lib.elmm_destroy, ctypes.c_void_p))
+s._h = None
+print("ok")
+"""
+
+OWNER = """
+#include <cstdlib>
+static void *handle;
+static int (*destroy)(void *);
+struct Owner {
+  ~Owner() {
+    if (destroy && destroy(handle)) std::_Exit(4);
+  }
+};
+static Owner owner;
+extern "C" void own(void *h, int (*d)(void *)) {
+  handle = h;
+  destroy = d;
+}
+"""
+
 
 def _run(tmp_path, script, arg):
     lib = str(tmp_path / "libhip_standin.so")
@@ -81,6 +109,14 @@ def _run(tmp_path, script, arg):
 @pytest.mark.parametrize("n", [8, 96])
 def test_transfers_of_a_handle_on_another_device(tmp_path, n):
     _run(tmp_path, TRANSFERS, str(n))
+
+
+def test_handle_destroyed_by_a_static_object(tmp_path):
+    src, lib = tmp_path / "owner.cpp", tmp_path / "libowner.so"
+    src.write_text(OWNER)
+    subprocess.run(["g++", "-shared", "-fPIC", str(src), "-o", str(lib)], check=True)
+    # loaded before the library's own static objects exist
+    _run(tmp_path, "ctypes.CDLL(sys.argv[3])\n" + AT_EXIT, str(lib))
 
 
 # a chunk fixed after a tuned handle, and before one (whose room for the SGS
