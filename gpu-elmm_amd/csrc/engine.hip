@@ -1768,8 +1768,7 @@ void Engine<T>::xfer_rows(E *d, const int lo[3], const int hi[3], int lb, const 
   const long nslab = (r1 - r0 + slab - 1) / slab;
   const int w = hi[0] - lo[0] + 1;
   const long hy = ext[0], hz = (long)ext[0] * ext[1];
-  auto convert = [&](E *buf, long s) {
-    const long b = r0 + s * slab, e = std::min(r1, b + slab);
+  auto convert = [&](E *buf, long b, long e) {  // rows b to e - 1
     if (whole) std::memset(buf, 0, (size_t)((e - b) * row_bytes));
     for (long r = b; r < e; r++) {
       const int j = (int)(r % per_k) - 2, k = (int)(r / per_k) - 2;
@@ -1782,23 +1781,30 @@ void Engine<T>::xfer_rows(E *d, const int lo[3], const int hi[3], int lb, const 
         for (int i = 0; i < w; i++) h[i] = (double)f[i];
     }
   };
+  const size_t span = (size_t)((r1 - r0) * row_bytes);
+  auto pageable = [&] {
+    std::unique_ptr<E[]> image(new E[span / sizeof(E)]);
+    E *dev = d + r0 * g.sy;
+    if (!whole) HIPCHK(hipMemcpy(image.get(), dev, span, hipMemcpyDeviceToHost));
+    convert(image.get(), r0, r1);
+    if (up) HIPCHK(hipMemcpy(dev, image.get(), span, hipMemcpyHostToDevice));
+  };
   // Small spans go through a pageable image in one copy each way: below some
   // 400 KiB the slots' events and the pins cost more than the copy engine
   // gives (16^3 FP64 16 against 21 us a field, 24^3 FP32 19 against 24, equal
   // at 36^3 FP32 of 440 KiB, 32^3 FP64 of 720 KiB 54 against 47)
-  const size_t span = (size_t)((r1 - r0) * row_bytes);
-  if (span <= 400 * 1024) {
-    std::unique_ptr<E[]> image(new E[span / sizeof(E)]);
-    E *dev = d + r0 * g.sy;
-    if (!whole) HIPCHK(hipMemcpy(image.get(), dev, span, hipMemcpyDeviceToHost));
-    convert(image.get(), 0);
-    if (up) HIPCHK(hipMemcpy(dev, image.get(), span, hipMemcpyHostToDevice));
-    return;
-  }
+  if (span <= 400 * 1024) return pageable();
   // two slots a thread, or the one it uses (a slot that is not in the pool
   // takes 0.6 ms to pin and 0.4 to free)
   const int per = nslab > nth ? 2 : 1;
-  PinnedPool::Slots slots(per * nth, (size_t)row_bytes);
+  std::unique_ptr<PinnedPool::Slots> pins;
+  try {
+    pins.reset(new PinnedPool::Slots(per * nth, (size_t)row_bytes));
+  } catch (const HipError &) {  // no memory to pin
+    (void)hipGetLastError();
+    return pageable();
+  }
+  PinnedPool::Slots &slots = *pins;
   auto task = [&](int t) {
     if (t >= nslab) return;  // few rows of more than a slot
     HostOpInherit inherit;
@@ -1822,7 +1828,7 @@ void Engine<T>::xfer_rows(E *d, const int lo[3], const int hi[3], int lb, const 
         copy(s + nth, q ^ 1, hipMemcpyDeviceToHost);
       }
       if (fetch || busy[q]) HIPCHK(hipEventSynchronize(slots.e[per * t + q]));
-      convert(static_cast<E *>(slots.p[per * t + q]), s);
+      convert(static_cast<E *>(slots.p[per * t + q]), r0 + s * slab, std::min(r1, r0 + (s + 1) * slab));
       if (up) {
         copy(s, q, hipMemcpyHostToDevice);
         busy[q] = true;

@@ -43,6 +43,7 @@ hipError_t hipFree(void *p) {
   return hipSuccess;
 }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+  if (std::getenv("STANDIN_NO_PINNED_MEMORY")) return hipErrorOutOfMemory;
   const hipError_t e = hipMalloc(p, n);
   std::lock_guard<std::mutex> lock(host_mu);
   if (e == hipSuccess) host.insert(*p);

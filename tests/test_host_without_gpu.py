@@ -105,9 +105,13 @@ def _run(tmp_path, script, arg):
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout + r.stderr
 
 
-# one task, on the caller's thread; several, on threads of their own
+# one task, on the caller's thread; several, on threads of their own; no memory
+# to be had for pinned slots
+@pytest.mark.parametrize("pinned", [True, False])
 @pytest.mark.parametrize("n", [8, 96])
-def test_transfers_of_a_handle_on_another_device(tmp_path, n):
+def test_transfers_of_a_handle_on_another_device(tmp_path, monkeypatch, n, pinned):
+    if not pinned:
+        monkeypatch.setenv("STANDIN_NO_PINNED_MEMORY", "1")
     _run(tmp_path, TRANSFERS, str(n))
 
 
