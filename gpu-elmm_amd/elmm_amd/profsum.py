@@ -36,8 +36,8 @@ def short(name):
     return name.replace("(anonymous namespace)::", "").replace("void ", "").split("(")[0]
 
 
-COUNTER_KERNELS = ("k_momentum_zm", "k_scalar_zm", "k_sgs_zm", "k_sgs<", "k_projection", "k_fft_x_fwd",
-                   "k_fft_x_inv", "k_fft_y", "k_solve_z")
+COUNTER_KERNELS = ("k_momentum_zm", "k_momentum<", "k_scalar_zm", "k_sgs_zm", "k_sgs<", "k_surface", "k_projection",
+                   "k_fft_x_fwd", "k_fft_x_inv", "k_fft_y", "k_solve_z")
 
 # Per dispatch a counter has one value per hardware instance (shader engine,
 # XCD...): SQ and TCC counters are summed over instances, GRBM ones (cycles
